@@ -55,14 +55,15 @@ struct SolverState {
     int32_t nonfinite;
     int32_t xit;       // updates already applied to x (the single-grid loop adds
                        // alpha*p to x in the next search, so x lags while xit < iter)
-    int32_t pad[2];
+    int32_t stalled;   // a cluster solve was abandoned: the solution is not to be used
+    int32_t pad;
 };
 
 // The solve has ended (stop test, iteration limit, non-finite value, or no
 // iteration allowed at all): launches that act on the solution are gated on
 // this, so they can be enqueued before the host knows whether the solve ended.
 __device__ __forceinline__ bool solve_finished(const SolverState* st) {
-    return st->done || st->iter >= st->max_iter;
+    return (st->done || st->iter >= st->max_iter) && !st->stalled;
 }
 
 // Times every launch of one named kernel with HIP events on the context's

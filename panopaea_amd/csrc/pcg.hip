@@ -14,6 +14,9 @@
 //
 // Arithmetic: fields in T, dot products accumulated in FP64, alpha/beta in
 // FP64, x/r/p updates formed in FP64 and rounded once to T.
+#include <cstdlib>
+
+#include "cg_cluster.hpp"
 #include "mg.hpp"
 #include "mg_device.hpp"
 #include "solver_device.hpp"
@@ -149,6 +152,9 @@ struct Solver {
     // `auxiliary` holds both (pcg.rs:51,65)
     T *x, *r, *aux, *p, *q;
     int it;  // iterations enqueued in this solve
+    ClPlan cl;           // the one-kernel loop (cl.wgs == 0: the launches)
+    ClSlots* slots;
+    unsigned spin;
 };
 
 // Entries of each partial-sum array: one per flat block, two per tile (the
@@ -164,7 +170,8 @@ static int solver_partials(const Dims& D, bool rb) {
 
 size_t pcg_workspace_bytes(const Dims& D) {
     auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
-    return al(sizeof(SolverState)) + 2 * al((size_t)solver_partials(D, false) * sizeof(double));
+    return al(sizeof(SolverState)) + 2 * al((size_t)solver_partials(D, false) * sizeof(double)) +
+           (cl_plan(D, sizeof(double)).wgs || cl_plan(D, sizeof(float)).wgs ? al(kClCopies * sizeof(ClSlots)) : 0);
 }
 
 // The parameter checks of solver_setup (no device work, no allocation).
@@ -213,6 +220,18 @@ static pano_status solver_setup(Ctx* c, const Dims& D, const pano_pcg_params* P,
     S->cfg.round_f32 = sizeof(T) == 4;
     int rm = P->remove_mean;
     S->cfg.remove_mean = rm < 0 ? (D.bc == 0) : rm;
+    // The one-kernel loop: identity and Jacobi solves whose cells fit the
+    // cluster. A kernel timer times the launches, so they run while one is set.
+    const char* cl = getenv("PANO_CG_CLUSTER");  // 0: off, 1: polls give up at once
+    S->cl = ClPlan();
+    S->spin = cl && cl[0] == '1' ? 1 : kClSpin;
+    if (!S->rb && P->max_iterations > 0 && c->timer.name.empty() && !(cl && cl[0] == '0'))
+        S->cl = cl_plan(D, sizeof(T), c->num_cu);
+    if (S->cl.wgs) {
+        void* sl;
+        PANO_CHECK(c->workspace("cl_slots", kClCopies * sizeof(ClSlots), &sl));
+        S->slots = (ClSlots*)sl;
+    }
     return PANO_OK;
 }
 
@@ -452,9 +471,28 @@ static pano_status solver_loop(Solver<T>* S, int max_iterations, int every, cons
     c->timer.solve = -1;
     return PANO_OK;
 }
-template <typename T>
-static pano_status solver_loop(Solver<T>* S, int max_iterations, int every, const std::string* key) {
-    return solver_loop<T>(S, max_iterations, every, key, []() { return PANO_OK; });
+
+// start() (the right-hand side into S->r, then solver_init), the loop, epi().
+// Where the cells fit the cluster the loop is one kernel; if that kernel was
+// abandoned (its workgroups did not all run together) everything starts over
+// with the launches: epi's kernels were no-ops then (solve_finished).
+template <typename T, typename Start, typename Epi>
+static pano_status solver_run(Solver<T>* S, int max_iterations, int every, const std::string* key, Start&& start,
+                              Epi&& epi) {
+    Ctx* c = S->c;
+    PANO_CHECK(start());
+    if (S->cl.wgs) {
+        const ClReserve cus(c->device, S->cl.wgs, c->num_cu);
+        PANO_CHECK(cl_solve<T>(c, S->D, S->cl, S->precond == PANO_PRECOND_JACOBI, S->x, S->r, S->p, S->aux, S->dt,
+                               S->mask, S->st, S->slots, S->spin));
+        PANO_CHECK(epi());
+        PANO_HIP(hipMemcpyAsync(&c->host_state[0], S->st, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
+        PANO_HIP(hipStreamSynchronize(c->stream));
+        c->timer.solve = -1;
+        if (!c->host_state[0].stalled) return PANO_OK;
+        PANO_CHECK(start());
+    }
+    return solver_loop<T>(S, max_iterations, every, key, epi);
 }
 
 // Key of the iteration-count hint: the problem shape and solver settings.
@@ -495,17 +533,20 @@ pano_status pcg_solve(Ctx* c, const Dims& D, const pano_pcg_params* P, T* x, con
         void* xr;
         PANO_CHECK(c->workspace("pcg_x_rb", (size_t)S.n * sizeof(T), &xr));
         S.x = (T*)xr;
-        L3((k_to_rb<T>), Gn, D, Gn, S.r, b);
     } else {
         S.x = x;
-        PANO_HIP(hipMemcpyAsync(S.r, b, (size_t)S.n * sizeof(T), hipMemcpyDeviceToDevice, c->stream));
     }
-    PANO_CHECK(solver_init<T>(&S, P->max_iterations));
+    auto start = [&]() -> pano_status {
+        if (S.rb) L3((k_to_rb<T>), Gn, D, Gn, S.r, b);
+        else PANO_HIP(hipMemcpyAsync(S.r, b, (size_t)S.n * sizeof(T), hipMemcpyDeviceToDevice, c->stream));
+        return solver_init<T>(&S, P->max_iterations);
+    };
+    auto epi = []() -> pano_status { return PANO_OK; };
     if (no_host_alloc) {
-        PANO_CHECK(solver_loop<T>(&S, P->max_iterations, P->check_every, nullptr));
+        PANO_CHECK(solver_run<T>(&S, P->max_iterations, P->check_every, nullptr, start, epi));
     } else {
         const std::string key = hint_key(D, P, sizeof(T));
-        PANO_CHECK(solver_loop<T>(&S, P->max_iterations, P->check_every, &key));
+        PANO_CHECK(solver_run<T>(&S, P->max_iterations, P->check_every, &key, start, epi));
     }
     if (S.rb) {
         L3((k_from_rb<T>), Gn, D, Gn, x, S.x);
@@ -592,21 +633,23 @@ static pano_status fluid_step(Ctx* c, const Dims& D, const pano_step_params* P, 
     const bool rhs_fused = !S.cfg.remove_mean;
     T* x0 = rhs_fused ? S.x : nullptr;
     double* pm = rhs_fused ? S.part1 : nullptr;
-    if (S.rb) {
-        if (D.d > 1) L3((k_neg_div_to<T, 3, REDBLACK>), Gd, D, Gd, S.r, v, x0, pm);
-        else L3((k_neg_div_to<T, 2, REDBLACK>), Gd, D, Gd, S.r, v, x0, pm);
-    } else {
-        if (D.d > 1) L3((k_neg_div_to<T, 3, NATURAL>), Gd, D, Gd, S.r, v, x0, pm);
-        else L3((k_neg_div_to<T, 2, NATURAL>), Gd, D, Gd, S.r, v, x0, pm);
-    }
-    PANO_HIP(hipGetLastError());
-    PANO_CHECK(solver_init<T>(&S, pp.max_iterations, rhs_fused ? (int)Gd.nb : 0));
+    auto start = [&]() -> pano_status {
+        if (S.rb) {
+            if (D.d > 1) L3((k_neg_div_to<T, 3, REDBLACK>), Gd, D, Gd, S.r, v, x0, pm);
+            else L3((k_neg_div_to<T, 2, REDBLACK>), Gd, D, Gd, S.r, v, x0, pm);
+        } else {
+            if (D.d > 1) L3((k_neg_div_to<T, 3, NATURAL>), Gd, D, Gd, S.r, v, x0, pm);
+            else L3((k_neg_div_to<T, 2, NATURAL>), Gd, D, Gd, S.r, v, x0, pm);
+        }
+        PANO_HIP(hipGetLastError());
+        return solver_init<T>(&S, pp.max_iterations, rhs_fused ? (int)Gd.nb : 0);
+    };
     const std::string key = hint_key(D, &pp, sizeof(T));
     // the loop's epilogue: u += dt d0_dual(p), closed walls zeroed; the x
     // component's pass also writes the pressure out in natural layout (gated
     // on the finished solve: the loop may enqueue it before it knows)
     const SolverState* gate = S.st;
-    PANO_CHECK(solver_loop<T>(&S, pp.max_iterations, pp.check_every, &key, [&]() -> pano_status {
+    PANO_CHECK(solver_run<T>(&S, pp.max_iterations, pp.check_every, &key, start, [&]() -> pano_status {
         if (S.rb) return launch_project_rb<T>(c, D, P->dt, vel_out, S.x, pressure, gate);
         return launch_project<T>(c, D, P->dt, vel_out, S.x, pressure, gate);
     }));
@@ -758,7 +801,7 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
         if (hs[1].done) break;
         // inner FP32 solve A e = r to the inner relative tolerance
         PANO_CHECK(solver_init<float>(&S, ip.max_iterations));
-        PANO_CHECK(solver_loop<float>(&S, ip.max_iterations, ip.check_every, &key));
+        PANO_CHECK(solver_loop<float>(&S, ip.max_iterations, ip.check_every, &key, []() { return PANO_OK; }));
         if (hs[0].nonfinite) return fail(PANO_ERR_NONFINITE, "non-finite value in the inner solve");
         inner_total += hs[0].iter;
         ++outer;
