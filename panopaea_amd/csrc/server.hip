@@ -10,12 +10,17 @@
 // over every admitted request. The launches of each phase go through
 // BatchCore, so a request's arithmetic and reduction order are those of the
 // request alone.
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <chrono>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <map>
 #include <memory>
+#include <system_error>
+#include <thread>
 #include <unordered_map>
 
 #include "batch.hpp"
@@ -68,11 +73,95 @@ private:
     int64_t used_ = 0;
 };
 
+// memcpy of large host ranges by a few threads. One thread copies into memory
+// it touches for the first time at 10 to 14 GB/s (page faults), four at three
+// times that. Threads that cannot be started leave their part to the caller.
+constexpr size_t kParCopyMin = size_t(4) << 20;
+static void par_copy(char* dst, const char* src, size_t n) {
+    constexpr int N = 4;
+    if (n < kParCopyMin) {
+        memcpy(dst, src, n);
+        return;
+    }
+    const size_t part = ((n / N + 4095) / 4096) * 4096;
+    std::thread th[N - 1];
+    for (int i = 1; i < N; ++i) {
+        const size_t a = std::min(n, i * part), b = i == N - 1 ? n : std::min(n, (i + 1) * part);
+        try {
+            th[i - 1] = std::thread([=] { memcpy(dst + a, src + a, b - a); });
+        } catch (const std::system_error&) {
+            memcpy(dst + a, src + a, b - a);
+        }
+    }
+    memcpy(dst, src, std::min(n, part));
+    for (std::thread& t : th)
+        if (t.joinable()) t.join();
+}
+
+// Host blocks for the velocities of queued requests. A block that a request
+// gives back is kept for the next one, up to kKeep bytes: a new allocation of
+// this size is page faults on its first write (the copy at submit took 190 ms
+// for 0.9 GB into new vectors). Blocks are huge-page advised.
+class HostPool {
+public:
+    ~HostPool() {
+        for (auto& b : free_) ::free(b.second);
+    }
+    // a block of at least n bytes (nullptr: no memory); *cap its size
+    void* take(size_t n, size_t* cap) {
+        auto it = free_.lower_bound(n);
+        if (it != free_.end() && it->first <= 2 * n + kAlign) {
+            void* p = it->second;
+            *cap = it->first;
+            kept_ -= it->first;
+            free_.erase(it);
+            return p;
+        }
+        *cap = (n + kAlign - 1) / kAlign * kAlign;
+        void* p = nullptr;
+        if (posix_memalign(&p, kAlign, *cap) != 0) return nullptr;
+        (void)madvise(p, *cap, MADV_HUGEPAGE);
+        return p;
+    }
+    void give(void* p, size_t cap) {
+        if (kept_ + cap > kKeep) {
+            ::free(p);
+            return;
+        }
+        kept_ += cap;
+        free_.emplace(cap, p);
+    }
+
+private:
+    static constexpr size_t kAlign = size_t(2) << 20, kKeep = size_t(1) << 30;
+    std::multimap<size_t, void*> free_;
+    size_t kept_ = 0;
+};
+
+// A block of the pool, given back when it goes.
+struct HostBlock {
+    HostPool* pool = nullptr;
+    void* p = nullptr;
+    size_t cap = 0;
+    HostBlock() = default;
+    HostBlock(HostPool* pl, size_t n) : pool(pl) { p = pl->take(n, &cap); }
+    HostBlock(HostBlock&& o) noexcept : pool(o.pool), p(o.p), cap(o.cap) { o.p = nullptr; }
+    HostBlock& operator=(HostBlock&& o) noexcept {
+        std::swap(pool, o.pool);
+        std::swap(p, o.p);
+        std::swap(cap, o.cap);
+        return *this;
+    }
+    ~HostBlock() {
+        if (p) pool->give(p, cap);
+    }
+};
+
 struct Request {
     int64_t id = 0;
     pano_grid pg;            // f32 grid description
     HGrid g;
-    std::vector<float> faces;        // host velocity until admission (empty: generate)
+    HostBlock faces;                 // host velocity until its upload has run (empty: generate)
     std::vector<double> gen_tab;     // host generator tables until the upload has run
     uint64_t seed = 0;
     int n_modes = 0;
@@ -89,6 +178,10 @@ struct Server {
     pano_server_params P;
     char* arena = nullptr;
     RangeAlloc alloc;
+    HostPool pool;                      // outlives the requests below
+    std::vector<HostBlock> uploading;   // blocks whose upload the stream may still read
+    char* fetch_stage = nullptr;        // pinned, two halves of kFetchChunk bytes
+    hipEvent_t fetch_ev[2] = {nullptr, nullptr};
     BatchCore core_all, core_new, core_done;
     SolverState* hstates = nullptr;  // pinned
     std::vector<SolveCfg> hcfg;
@@ -135,6 +228,50 @@ static pano_status stage_upload(Server* S, void* dst, const void* src, size_t n)
     return PANO_OK;
 }
 
+// The pressure of a solved request (red-black pairs) in natural order.
+__global__ __launch_bounds__(256) void k_rb_to_nat(Dims D, Grid3 G, float* dst, const float* src) {
+    int x, y, z, L;
+    tile_xyz(G, x, y, z, L);
+    if (x >= D.w || y >= D.h) return;
+    stx(dst, cell_index(D, z, y, x), ldx(src, rb_index(D, z, y, x)));
+}
+
+// Device range to (pageable) host memory. Large ranges go through two pinned
+// halves: the next chunk's copy runs while a few threads move the last one to
+// its place (a plain copy into new memory: 10 GB/s).
+constexpr size_t kFetchChunk = size_t(8) << 20;
+static pano_status fetch_range(Server* S, char* dst, const char* src, size_t n) {
+    hipStream_t st = S->c->stream;
+    if (n >= kParCopyMin && !S->fetch_stage) {
+        if (hipHostMalloc((void**)&S->fetch_stage, 2 * kFetchChunk) != hipSuccess) {
+            (void)hipGetLastError();
+            S->fetch_stage = nullptr;
+            return fail(PANO_ERR_OOM, "pinned staging of %zu bytes", 2 * kFetchChunk);
+        }
+        for (hipEvent_t& e : S->fetch_ev) PANO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    if (n < kParCopyMin) {
+        PANO_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
+        PANO_HIP(hipStreamSynchronize(st));
+        return PANO_OK;
+    }
+    const size_t chunks = (n + kFetchChunk - 1) / kFetchChunk;
+    auto size_of = [&](size_t k) { return std::min(kFetchChunk, n - k * kFetchChunk); };
+    auto enqueue = [&](size_t k) -> pano_status {
+        PANO_HIP(hipMemcpyAsync(S->fetch_stage + (k & 1) * kFetchChunk, src + k * kFetchChunk, size_of(k),
+                                hipMemcpyDeviceToHost, st));
+        PANO_HIP(hipEventRecord(S->fetch_ev[k & 1], st));
+        return PANO_OK;
+    };
+    PANO_CHECK(enqueue(0));
+    for (size_t k = 0; k < chunks; ++k) {
+        if (k + 1 < chunks) PANO_CHECK(enqueue(k + 1));
+        PANO_HIP(hipEventSynchronize(S->fetch_ev[k & 1]));
+        par_copy(dst + k * kFetchChunk, S->fetch_stage + (k & 1) * kFetchChunk, size_of(k));
+    }
+    return PANO_OK;
+}
+
 static std::vector<HGrid> grids_of(const std::vector<Request*>& v, std::vector<int>& ids) {
     std::vector<HGrid> g;
     ids.clear();
@@ -162,7 +299,7 @@ static pano_status admit_at(Server* S, Request* r, int64_t off, std::vector<Requ
 // pinned staging, upload or generator launch) the range and the solver slot
 // are given back and the request stays queued as it was.
 static pano_status admit(Server* S, Request* r, std::vector<Request*>& fresh) {
-    const int64_t need = r->bytes + (r->faces.empty() ? al256(r->tab_bytes) : 0);
+    const int64_t need = r->bytes + (r->faces.p ? 0 : al256(r->tab_bytes));
     const int64_t off = S->alloc.alloc(need);
     if (off < 0) return PANO_NOT_CONVERGED;  // does not fit now
     const pano_status st = admit_at(S, r, off, fresh);
@@ -180,7 +317,7 @@ static pano_status admit_at(Server* S, Request* r, int64_t off, std::vector<Requ
     Ctx* c = S->c;
     r->off = off;
     PANO_CHECK(request_layout(S, r, off));
-    r->tab_off = r->faces.empty() ? off + al256(r->bytes) : -1;
+    r->tab_off = r->faces.p ? -1 : off + al256(r->bytes);
     r->slot = S->free_slots.back();
     S->free_slots.pop_back();
     r->g.sidx = r->slot;
@@ -193,14 +330,14 @@ static pano_status admit_at(Server* S, Request* r, int64_t off, std::vector<Requ
     cf.round_f32 = 1;
     PANO_CHECK(stage_upload(S, S->core_all.cfgs + r->slot, &cf, sizeof(SolveCfg)));
     float* u = reinterpret_cast<float*>(S->arena + r->g.o_u[0]);
-    if (!r->faces.empty()) {
-        PANO_CHECK(stage_upload(S, u, r->faces.data(), r->faces.size() * sizeof(float)));
+    if (r->faces.p) {
+        PANO_HIP(hipMemcpyAsync(u, r->faces.p, r->g.faces * sizeof(float), hipMemcpyHostToDevice, c->stream));
+        S->uploading.push_back(std::move(r->faces));
     } else {
         double* dtab = reinterpret_cast<double*>(S->arena + r->tab_off);
         PANO_CHECK(stage_upload(S, dtab, r->gen_tab.data(), r->gen_tab.size() * sizeof(double)));
         PANO_CHECK(gen_faces_enqueue(c, &r->pg, r->n_modes, r->amplitude, dtab, u));
     }
-    std::vector<float>().swap(r->faces);
     std::vector<double>().swap(r->gen_tab);
     r->state = PANO_REQ_ADMITTED;
     r->t_admit = S->now();
@@ -212,6 +349,7 @@ static pano_status server_tick(Server* S) {
     Ctx* c = S->c;
     PANO_HIP(hipStreamSynchronize(c->stream));
     S->stage_used = 0;
+    S->uploading.clear();
     // (1) the previous tick's retirements have completed
     double t = S->now();
     for (Request* r : S->retiring) {
@@ -362,6 +500,9 @@ pano_status pano_server_destroy(pano_server h) {
     if (S->arena) (void)hipFree(S->arena);
     if (S->hstates) (void)hipHostFree(S->hstates);
     if (S->stage) (void)hipHostFree(S->stage);
+    if (S->fetch_stage) (void)hipHostFree(S->fetch_stage);
+    for (hipEvent_t e : S->fetch_ev)
+        if (e) (void)hipEventDestroy(e);
     delete h;
     return PANO_OK;
 }
@@ -385,7 +526,10 @@ pano_status pano_server_submit(pano_server h, const pano_server_request* q, int6
     r->g.dt = q->grid.dt;
     PANO_CHECK(request_layout(S, r.get(), 0));
     if (q->faces) {
-        r->faces.assign(q->faces, q->faces + r->g.faces);
+        const size_t n = (size_t)r->g.faces * sizeof(float);
+        r->faces = HostBlock(&S->pool, n);
+        if (!r->faces.p) return fail(PANO_ERR_OOM, "host memory for a request's velocity (%zu bytes)", n);
+        par_copy((char*)r->faces.p, (const char*)q->faces, n);
     } else {
         r->seed = q->seed;
         r->n_modes = q->n_modes;
@@ -455,27 +599,19 @@ pano_status pano_server_fetch(pano_server h, int64_t id, float* faces, float* pr
     if (it == S->reqs.end()) return fail(PANO_ERR_INVALID, "unknown request %lld", (long long)id);
     const Request* r = it->second.get();
     if (r->state != PANO_REQ_DONE) return fail(PANO_ERR_INVALID, "request %lld is not done", (long long)id);
-    hipStream_t st = S->c->stream;
-    if (faces)
-        PANO_HIP(hipMemcpyAsync(faces, S->arena + r->g.o_u[0], r->g.faces * sizeof(float), hipMemcpyDeviceToHost,
-                                st));
-    std::vector<float> rb;
+    Ctx* c = S->c;
+    PANO_HIP(hipSetDevice(c->device));
     if (pressure) {
-        rb.resize(r->g.cells);
-        PANO_HIP(hipMemcpyAsync(rb.data(), S->arena + r->g.o_x, r->g.cells * sizeof(float), hipMemcpyDeviceToHost,
-                                st));
-    }
-    PANO_HIP(hipStreamSynchronize(st));
-    if (pressure) {  // red-black order -> natural order
+        // red-black -> natural order in the request's residual field, which a
+        // solved request no longer needs
         const Dims& D = r->g.D;
-        int64_t wh = D.w >> 1, n2 = (int64_t)D.d * D.h * wh;
-        for (int z = 0; z < D.d; ++z)
-            for (int y = 0; y < D.h; ++y)
-                for (int x = 0; x < D.w; ++x) {
-                    int64_t c = (x + y + z) & 1;
-                    pressure[((int64_t)z * D.h + y) * D.w + x] = rb[c * n2 + ((int64_t)z * D.h + y) * wh + (x >> 1)];
-                }
+        const Grid3 G = grid3(D.w, D.h, D.d);
+        hipLaunchKernelGGL(k_rb_to_nat, dim3(G.nb), dim3(kTX, kTY), 0, c->stream, D, G,
+                           (float*)(S->arena + r->g.o_r), (const float*)(S->arena + r->g.o_x));
+        PANO_HIP(hipGetLastError());
     }
+    if (faces) PANO_CHECK(fetch_range(S, (char*)faces, S->arena + r->g.o_u[0], r->g.faces * sizeof(float)));
+    if (pressure) PANO_CHECK(fetch_range(S, (char*)pressure, S->arena + r->g.o_r, r->g.cells * sizeof(float)));
     return PANO_OK;
 }
 

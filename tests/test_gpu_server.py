@@ -134,3 +134,37 @@ def run_alone_grid(g, seed):
     out = S.fetch(rid)
     S.close()
     return out
+
+
+@pytest.mark.parametrize("dims,bc", [((1024, 1024), (0,) * 6),              # pressure exactly 4 MiB, faces past 8 MiB
+                                     ((1024, 1016), (0, 1, 0, 0, 0, 0)),    # pressure just below 4 MiB
+                                     ((104, 168, 176), (0, 0, 0, 0, 0, 1)),  # several chunks and a remainder
+                                     ((16, 24), (0,) * 6)])
+def test_gpu_server_host_velocity_and_fetch(dims, bc):
+    """A host velocity gives the bits of the same field generated on the
+    device, and the fetched velocity is u + dt d0*(p) of the fetched pressure
+    in natural order (f32, the projection's own expression), for sizes on both
+    sides of the copies' chunk limits. Two requests share the server, the
+    second one's host block was the first one's."""
+    print("server host velocity", dims, flush=True)
+    g = dict(dims=dims, dt=0.5 / dims[-1], bc=bc)
+    grid = (pa.Grid2d if len(dims) == 2 else pa.Grid3d)(dims, np.float32, bc=bc)
+    nm, km = modes(g)
+    S = pa.Server(hbm_budget=2 << 30, max_active=4, mg_levels=3)
+    for seed in (3, 4):
+        u = pa.gen_bandlimited_faces(grid, seed, nm, km)
+        a = S.submit(g, faces=u)
+        S.run_until_idle()
+        b = S.submit(g, seed=seed, n_modes=nm, k_max=km)
+        S.run_until_idle()
+        (fa, p), (fb, q) = S.fetch(a), S.fetch(b)
+        assert np.array_equal(fa, fb) and np.array_equal(p, q)
+        fc, pc = S.fetch(a)
+        assert np.array_equal(fa, fc) and np.array_equal(p, pc)
+        S.release(a)
+        S.release(b)
+        P, dt = p.reshape(dims), np.float32(g["dt"])
+        _, _, ux = grid.split_faces(u)
+        _, _, vx = grid.split_faces(fa)
+        assert np.array_equal(vx[..., 1:-1], ux[..., 1:-1] + dt * (P[..., :-1] - P[..., 1:]))
+    S.close()
