@@ -401,26 +401,31 @@ __global__ __launch_bounds__(256) void kb_fdm_zcol(FTab T, char* A, const Solver
                   F.s, 1e-10);
 }
 
-// 2D coarsest level: row pass 0 (forward x) or 2 (inverse x) over row blocks.
-__global__ __launch_bounds__(256) void kb_fdm2_rows(FTab T, char* A, int pass, const SolverState* st) {
+// 2D coarsest level of the grids that one workgroup solves.
+__global__ __launch_bounds__(kFdm2Threads) void kb_fdm2_one(FTab T, char* A, const SolverState* st) {
     extern __shared__ double fdm_lds[];
     FDM_ENTRY(T);
     if (st[F.sidx].done) return;
-    int blk = blockIdx.x - F.start;
-    if (pass == 0)
-        fdm2_rows_body<float, double>(fdm_lds, F.nx, F.ny, blk, 0, (const float*)fld<float>(A, F.o_r),
-                                      fld<double>(A, F.o_t0), F.Vx);
-    else
-        fdm2_rows_body<double, float>(fdm_lds, F.nx, F.ny, blk, 1, (const double*)fld<double>(A, F.o_t0),
-                                      fld<float>(A, F.o_z), F.Vx);
+    fdm2_one_body<float, float>(fdm_lds, F.nx, F.ny, (const float*)fld<float>(A, F.o_r), fld<float>(A, F.o_z), F.Vx,
+                                F.Vy, F.lx, F.ly, F.s, 1e-10);
 }
 
-// 2D coarsest level: column pass over column blocks.
-__global__ __launch_bounds__(256) void kb_fdm2_cols(FTab T, char* A, const SolverState* st) {
-    extern __shared__ double fdm_lds[];
+// 2D coarsest level of the other grids: product `pass` of fdm2_tile_body.
+__global__ __launch_bounds__(256) void kb_fdm2_tile(FTab T, char* A, int pass, const SolverState* st) {
+    __shared__ double lds[1024];
     FDM_ENTRY(T);
     if (st[F.sidx].done) return;
-    fdm2_cols_body(fdm_lds, F.nx, F.ny, blockIdx.x - F.start, fld<double>(A, F.o_t0), F.Vy, F.lx, F.ly, F.s, 1e-10);
+    const int t = blockIdx.x - F.start;
+    double *t0 = fld<double>(A, F.o_t0), *t1 = fld<double>(A, F.o_t1);
+    if (pass == 0)
+        fdm2_tile_body<float, double>(lds, F.nx, F.ny, t, 0, (const float*)fld<float>(A, F.o_r), t0, F.Vx, F.Vy, F.lx,
+                                      F.ly, F.s, 1e-10);
+    else if (pass == 3)
+        fdm2_tile_body<double, float>(lds, F.nx, F.ny, t, 3, (const double*)t0, fld<float>(A, F.o_z), F.Vx, F.Vy,
+                                      F.lx, F.ly, F.s, 1e-10);
+    else
+        fdm2_tile_body<double, double>(lds, F.nx, F.ny, t, pass, (const double*)(pass == 1 ? t0 : t1),
+                                       pass == 1 ? t1 : t0, F.Vx, F.Vy, F.lx, F.ly, F.s, 1e-10);
 }
 
 // ---- host side -------------------------------------------------------------------------------
@@ -617,8 +622,8 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
     }
     plane_.h.clear();
     zcol_.h.clear();
-    rows2_.h.clear();
-    cols2_.h.clear();
+    one2_.h.clear();
+    tile2_.h.clear();
     levels_ = ids.empty() ? 0 : grids[ids[0]].levels;
     any3d_ = false;
     for (int l = 0; l < 16; ++l) split_first_[l] = false;
@@ -626,7 +631,7 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
     int srbs[16] = {0}, stb[16][kTbConfigs] = {}, sap = 0;
     int srsd[16] = {0}, srr2[16] = {0};
     std::vector<std::pair<int, int>> dot_src;  // per grid: (config + 1 or 0 for half-sweeps, entry index) at level 0
-    int srow = 0, scol = 0;
+    int sone = 0, stile = 0;
     size_t maxp = 0;
     for (int id : ids) {
         const HGrid& g = grids[id];
@@ -801,6 +806,7 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
                 F.o_r = g.o_rl[l];
                 F.o_z = g.o_zl[l];
                 F.o_t0 = g.o_t0;
+                F.o_t1 = g.o_res;  // free during the coarsest solve, 16 bytes and more per coarse cell
                 if (D.d > 1) {
                     F.start = splane;
                     F.nblk = L.d;
@@ -812,15 +818,13 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
                     szcol += Z.nblk;
                     zcol_.h.push_back(Z);
                 } else {
-                    F.start = srow;
-                    F.nblk = (L.h + fdm2_rows_per(L.w) - 1) / fdm2_rows_per(L.w);
-                    srow += F.nblk;
-                    rows2_.h.push_back(F);
-                    BFdm Cc = F;
-                    Cc.start = scol;
-                    Cc.nblk = (L.w + fdm2_cols_per(L.h) - 1) / fdm2_cols_per(L.h);
-                    scol += Cc.nblk;
-                    cols2_.h.push_back(Cc);
+                    // one workgroup, or the 16 x 16 tiles of four launches
+                    const bool one = fdm2_one(L.w, L.h);
+                    int& first = one ? sone : stile;
+                    F.start = first;
+                    F.nblk = one ? 1 : ((L.w + 15) / 16) * ((L.h + 15) / 16);
+                    first += F.nblk;
+                    (one ? one2_ : tile2_).h.push_back(F);
                 }
             }
             s *= 0.25;
@@ -847,14 +851,13 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
         }
     }
     fdm_lds_ = kFdmLdsBytes;
-    // 2D coarsest passes: the largest need of the grids in the launch
-    rows2_lds_ = cols2_lds_ = 0;
-    for (const BFdm& F : rows2_.h) rows2_lds_ = std::max(rows2_lds_, fdm2_rows_lds(F.nx));
-    for (const BFdm& F : cols2_.h) cols2_lds_ = std::max(cols2_lds_, fdm2_cols_lds(F.ny));
+    // 2D coarsest level: the largest need of the grids in the launch
+    one2_lds_ = 0;
+    for (const BFdm& F : one2_.h) one2_lds_ = std::max(one2_lds_, fdm2_one_lds(F.nx, F.ny));
     // pack every table into the staging buffer, then one copy
     size_t total = table_bytes(nat_) + table_bytes(fx_) + table_bytes(fy_) + table_bytes(fz_) + table_bytes(flat_) +
                    table_bytes(ap_) +
-                   table_bytes(plane_) + table_bytes(zcol_) + table_bytes(rows2_) + table_bytes(cols2_);
+                   table_bytes(plane_) + table_bytes(zcol_) + table_bytes(one2_) + table_bytes(tile2_);
     for (int p = 0; p < 2; ++p)
         total += table_bytes(div_[p]) + table_bytes(prc_[p]);
     for (int l = 0; l + 1 < levels_; ++l) {
@@ -900,8 +903,8 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
     PANO_CHECK(place(dot_));
     PANO_CHECK(place(plane_));
     PANO_CHECK(place(zcol_));
-    PANO_CHECK(place(rows2_));
-    PANO_CHECK(place(cols2_));
+    PANO_CHECK(place(one2_));
+    PANO_CHECK(place(tile2_));
     PANO_HIP(hipMemcpyAsync(tab_dev_, tab_host_, tab_used_, hipMemcpyHostToDevice, c->stream));
     PANO_CHECK(ensure_partials(std::max<size_t>(maxp, 1)));
     return PANO_OK;
@@ -1017,15 +1020,12 @@ pano_status BatchCore::vcycle(bool with_dot) {
         else BL(kb_resrestrict2<REDBLACK>, rr2_[l], arena, (const SolverState*)states);
         blk = sblk;
     }
-    if (!rows2_.h.empty()) {
-        const SolverState* cst = states;
-        hipLaunchKernelGGL(kb_fdm2_rows, dim3(rows2_.nbt), dim3(256), rows2_lds_, c->stream, rows2_.view(), arena, 0,
-                           cst);
-        hipLaunchKernelGGL(kb_fdm2_cols, dim3(cols2_.nbt), dim3(256), cols2_lds_, c->stream, cols2_.view(), arena,
-                           cst);
-        hipLaunchKernelGGL(kb_fdm2_rows, dim3(rows2_.nbt), dim3(256), rows2_lds_, c->stream, rows2_.view(), arena, 2,
-                           cst);
-    }
+    if (!one2_.h.empty())
+        hipLaunchKernelGGL(kb_fdm2_one, dim3(one2_.nbt), dim3(kFdm2Threads), one2_lds_, c->stream, one2_.view(), arena,
+                           (const SolverState*)states);
+    for (int pass = 0; pass < 4 && !tile2_.h.empty(); ++pass)
+        hipLaunchKernelGGL(kb_fdm2_tile, dim3(tile2_.nbt), dim3(256), 0, c->stream, tile2_.view(), arena, pass,
+                           (const SolverState*)states);
     if (!plane_.h.empty()) {
         const SolverState* cst = states;
         hipLaunchKernelGGL(kb_fdm_plane, dim3(plane_.nbt), dim3(256), fdm_lds_, c->stream, plane_.view(), arena, 0,

@@ -43,7 +43,7 @@ struct BFdm {
     int nx, ny, nz;
     const double *Vx, *Vy, *Vz, *lx, *ly, *lz;
     double s;
-    int64_t o_r, o_z, o_t0;  // arena byte offsets: coarse rhs (f32), solution (f32), FP64 temp
+    int64_t o_r, o_z, o_t0, o_t1;  // arena byte offsets: coarse rhs (f32), solution (f32), FP64 temps
 };
 
 // Device view of a launch table: entries sorted by first block, and their
@@ -161,7 +161,7 @@ private:
                            // (o[0] = z_l, o[1] = r_l, o[2] = r_{l+1})
     Table prl_[16];        // pair tiles of level l for the prolongation from l+1
     FdmTable plane_, zcol_;  // 3D coarsest solve
-    FdmTable rows2_, cols2_;  // 2D coarsest solve
+    FdmTable one2_, tile2_;  // 2D coarsest solve: one workgroup per grid / tiles of four products
     int levels_ = 0;
     bool any3d_ = false;
     bool split_first_[16] = {};  // first sweep as red cells + black half-sweep at this level
@@ -172,7 +172,7 @@ private:
     bool pro_ = true;
     int tb_base_[kTbConfigs] = {};  // first partial slot of each configuration's level-0 launch
     size_t fdm_lds_ = 0;
-    size_t rows2_lds_ = 0, cols2_lds_ = 0;  // dynamic LDS of the 2D coarsest passes
+    size_t one2_lds_ = 0;  // dynamic LDS of the one-workgroup 2D coarsest solve
     double* part0_ = nullptr;
     double* part1_ = nullptr;
     double* part2_ = nullptr;

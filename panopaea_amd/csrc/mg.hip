@@ -525,18 +525,21 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_plane_rc(Dims Df, Dims Dc, 
 }
 
 template <typename Tin, typename Tout>
-__global__ __launch_bounds__(256) void k_fdm2_rows(int nx, int ny, int inverse, const Tin* in, Tout* out,
-                                                   const double* Vx, const SolverState* st) {
-    if (st->done) return;
-    extern __shared__ double fdm_lds[];
-    fdm2_rows_body<Tin, Tout>(fdm_lds, nx, ny, blockIdx.x, inverse, in, out, Vx);
-}
-
-__global__ __launch_bounds__(256) void k_fdm2_cols(int nx, int ny, double* t, const double* Vy, const double* lx,
+__global__ __launch_bounds__(256) void k_fdm2_tile(int nx, int ny, int pass, const Tin* in, Tout* out,
+                                                   const double* Vx, const double* Vy, const double* lx,
                                                    const double* ly, double s, double eps, const SolverState* st) {
     if (st->done) return;
+    __shared__ double lds[1024];
+    fdm2_tile_body<Tin, Tout>(lds, nx, ny, blockIdx.x, pass, in, out, Vx, Vy, lx, ly, s, eps);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kFdm2Threads) void k_fdm2_one(int nx, int ny, const T* in, T* out, const double* Vx,
+                                                           const double* Vy, const double* lx, const double* ly,
+                                                           double s, double eps, const SolverState* st) {
+    if (st->done) return;
     extern __shared__ double fdm_lds[];
-    fdm2_cols_body(fdm_lds, nx, ny, blockIdx.x, t, Vy, lx, ly, s, eps);
+    fdm2_one_body<T, T>(fdm_lds, nx, ny, in, out, Vx, Vy, lx, ly, s, eps);
 }
 
 __global__ __launch_bounds__(kFdmThreads) void k_fdm_zcol(int nx, int ny, int nz, double* data, const double* Vz,
@@ -759,15 +762,21 @@ static pano_status coarse_solve(Ctx* c, MG<T>* m, T* z, const T* r, const Solver
     hipStream_t S = c->stream;
     const double *Vx = m->fdm_v[0], *Vy = m->fdm_v[1], *Vz = m->fdm_v[2];
     const double *lx = m->fdm_lam[0], *ly = m->fdm_lam[1], *lz = m->fdm_lam[2];
-    if (DIM == 2 && nx <= kFdmPlane && ny <= kFdmPlane) {
-        // rows (forward x), columns (y, divide, inverse y), rows (inverse x)
-        const size_t lr = fdm2_rows_lds(nx), lc = fdm2_cols_lds(ny);
-        unsigned nr = (unsigned)((ny + fdm2_rows_per(nx) - 1) / fdm2_rows_per(nx));
-        unsigned ncol = (unsigned)((nx + fdm2_cols_per(ny) - 1) / fdm2_cols_per(ny));
-        hipLaunchKernelGGL((k_fdm2_rows<T, double>), dim3(nr), dim3(256), lr, S, nx, ny, 0, r, t0, Vx, st);
-        hipLaunchKernelGGL(k_fdm2_cols, dim3(ncol), dim3(256), lc, S, nx, ny, t0, Vy, lx, ly, s, eps, st);
-        hipLaunchKernelGGL((k_fdm2_rows<double, T>), dim3(nr), dim3(256), lr, S, nx, ny, 1, (const double*)t0, z,
-                           Vx, st);
+    if (DIM == 2) {
+        if (fdm2_one(nx, ny)) {
+            hipLaunchKernelGGL((k_fdm2_one<T>), dim3(1), dim3(kFdm2Threads), fdm2_one_lds(nx, ny), S, nx, ny, r, z, Vx,
+                               Vy, lx, ly, s, eps, st);
+        } else {
+            const dim3 G((unsigned)(((nx + 15) / 16) * ((ny + 15) / 16)));
+            hipLaunchKernelGGL((k_fdm2_tile<T, double>), G, dim3(256), 0, S, nx, ny, 0, r, t0, Vx, Vy, lx, ly, s, eps,
+                               st);
+            hipLaunchKernelGGL((k_fdm2_tile<double, double>), G, dim3(256), 0, S, nx, ny, 1, (const double*)t0, t1, Vx,
+                               Vy, lx, ly, s, eps, st);
+            hipLaunchKernelGGL((k_fdm2_tile<double, double>), G, dim3(256), 0, S, nx, ny, 2, (const double*)t1, t0, Vx,
+                               Vy, lx, ly, s, eps, st);
+            hipLaunchKernelGGL((k_fdm2_tile<double, T>), G, dim3(256), 0, S, nx, ny, 3, (const double*)t0, z, Vx, Vy,
+                               lx, ly, s, eps, st);
+        }
         PANO_HIP(hipGetLastError());
         return PANO_OK;
     }
@@ -810,21 +819,14 @@ static pano_status coarse_solve(Ctx* c, MG<T>* m, T* z, const T* r, const Solver
     unsigned nb = blocks_for(n, kBlock);
     hipLaunchKernelGGL((k_fdm_axis<T, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 0, 0, r, t0, Vx, 0,
                        nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    if (DIM == 3) {
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 0, t0, t1, Vy,
-                           0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 0, t1, t0, Vz,
-                           1, lx, ly, lz, s, eps, st);
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 1, t0, t1, Vz,
-                           0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 1, t1, t0, Vy,
-                           0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    } else {
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 0, t0, t1, Vy,
-                           1, lx, ly, nullptr, s, eps, st);
-        hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 1, t1, t0, Vy,
-                           0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    }
+    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 0, t0, t1, Vy,
+                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
+    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 0, t1, t0, Vz,
+                       1, lx, ly, lz, s, eps, st);
+    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 1, t0, t1, Vz,
+                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
+    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 1, t1, t0, Vy,
+                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
     hipLaunchKernelGGL((k_fdm_axis<double, T>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 0, 1, t0, z, Vx, 0,
                        nullptr, nullptr, nullptr, 0.0, 0.0, st);
     PANO_HIP(hipGetLastError());

@@ -756,103 +756,173 @@ __device__ __forceinline__ void fdm_plane_body(double* lds, int nx, int ny, int 
         lds, nx, ny, mode, [src](int e) { return (double)src[e]; }, dst, Vx, Vy, lx, ly, s, eps);
 }
 
-// 2D coarsest level as three passes over lines, each output element summed in
-// the order of lds_axis (so the result equals fdm_plane_body mode 2):
-//  pass 0, rows: t[j,i] = sum_q Vx[q*nx+i] * r[j*nx+q]        (forward x)
-//  pass 1, columns: u[j,i] = sum_q Vy[q*ny+j] * t[q*nx+i]    (forward y),
-//          u /= s*(lx[i]+ly[j]) (0 on the null space), t[j,i] = sum_k Vy[j*ny+k] * u[k*nx+i]
-//  pass 2, rows: z[j,i] = sum_k Vx[i*nx+k] * t[j*nx+k]        (inverse x)
-// Rows per workgroup: fdm2_rows_per(nx); columns per workgroup: fdm2_cols_per(ny).
-__host__ __device__ inline int fdm2_rows_per(int nx) { return nx >= 256 ? 1 : 256 / nx; }
-__host__ __device__ inline int fdm2_cols_per(int ny) { return ny >= 256 ? 1 : 256 / ny; }
-// Dynamic LDS bytes of the passes: the workgroup's lines, then the eigenbasis
-// when it is staged (stage_basis), so small levels leave room for several
-// workgroups per CU.
-__host__ __device__ inline size_t fdm2_rows_lds(int nx) {
-    const size_t R = fdm2_rows_per(nx);
-    return (R * nx + (nx * nx <= kFdmVStage ? (size_t)nx * nx : 0)) * sizeof(double);
-}
-__host__ __device__ inline size_t fdm2_cols_lds(int ny) {
-    const size_t C = fdm2_cols_per(ny);
-    return (2 * C * ny + (ny * ny <= kFdmVStage ? (size_t)ny * ny : 0)) * sizeof(double);
+// ---- 2D coarsest level: four FP64 matrix products on the matrix cores ----------------
+// Z = Vy ((Vy^T (R Vx)) / (s (lx + ly))) Vx^T, with R, Z ny x nx. In 16 x 16
+// tiles of v_mfma_f64_16x16x4: a lane reads one entry of each operand per 16
+// products it takes part in, where a sum per thread read two entries per
+// product from LDS and was bound by those reads (128 x 128: 32.7 us in three
+// launches, 16.4 us in four now; the 64 coarsest grids of 8 x 8 to 64 x 64 of a
+// batch: 25 us in three launches, 11.3 us in one).
+using mfma_d4 = double __attribute__((ext_vector_type(4)));
+
+// acc += sum over q in [q0, q1) of fa(q) fb(q), fa/fb the lane's entries: A(row
+// lane % 16, q) and B(q, column lane % 16), q taking lane / 16 as its low part.
+// acc[v] is the entry (4 v + lane / 16, lane % 16). U steps' loads in flight.
+template <int U, typename FA, typename FB>
+__device__ __forceinline__ void mfma_tile(int q0, int q1, FA fa, FB fb, mfma_d4& acc) {
+    const int kq = (threadIdx.x & 63) >> 4;
+    for (int k0 = q0; k0 < q1; k0 += 4 * U) {
+        double a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int q = k0 + 4 * u + kq, qc = q < q1 ? q : q1 - 1;
+            const double x = fa(qc), y = fb(qc);
+            a[u] = q < q1 ? x : 0.0;
+            b[u] = q < q1 ? y : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
+    }
 }
 
-// rows [blk*R, blk*R + R) of pass 0 (Tin -> double t) or pass 2 (double t -> Tout); lds: R*nx doubles,
-// then the staged basis (fdm2_rows_lds)
+// One product of a solve too large for one workgroup: tile t of the output,
+// four waves with a quarter of the sum each (added in order through lds, 1024
+// doubles). pass 0: R Vx -> out; 1: (Vy^T in) / (s (lx + ly)) -> out (0 on the
+// null space); 2: Vy in -> out; 3: in Vx^T -> out.
 template <typename Tin, typename Tout>
-__device__ __forceinline__ void fdm2_rows_body(double* lds, int nx, int ny, int blk, int inverse, const Tin* src,
-                                               Tout* dst, const double* Vx) {
-    const int R = fdm2_rows_per(nx);
-    const int j0 = blk * R;
-    const int nr = min(R, ny - j0);
-    const int P = nr * nx;
-    // the rows and the basis in one round of loads (inverse: the transpose W,
-    // W[k*nx+i] = Vx[i*nx+k]), the basis when it fits (kFdmVStage)
-    const bool sv = nx * nx <= kFdmVStage;
-    const Tin* rows = src + (int64_t)j0 * nx;
-    double* vs = lds + R * nx;
-    if (inverse)
-        lds_fill2<1, 16>(
-            lds, P, [&](int e) { return (double)rows[e]; }, vs, sv ? nx * nx : 0,
-            [&](int e) {
-                const int q = e / nx, i = e - q * nx;
-                return Vx[i * nx + q];
-            });
-    else
-        lds_fill2<1, 16>(
-            lds, P, [&](int e) { return (double)rows[e]; }, vs, sv ? nx * nx : 0, [&](int e) { return Vx[e]; });
-    const double* W = inverse && sv ? vs : nullptr;
-    if (!inverse && sv) Vx = vs;
-    __syncthreads();
-    for (int e = threadIdx.x; e < P; e += blockDim.x) {
-        int jl = e / nx, i = e - jl * nx;
-        const double* a = lds + jl * nx;
-        double acc = 0.0;
-        if (W)
-            for (int k = 0; k < nx; ++k) acc += W[k * nx + i] * a[k];
-        else if (inverse)
-            for (int k = 0; k < nx; ++k) acc += Vx[i * nx + k] * a[k];
+__device__ __forceinline__ void fdm2_tile_body(double* lds, int nx, int ny, int t, int pass, const Tin* in, Tout* out,
+                                               const double* Vx, const double* Vy, const double* lx,
+                                               const double* ly, double s, double eps) {
+    const int gx = (nx + 15) >> 4, ti = t % gx, tj = t / gx;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15;
+    const int j = imin(tj * 16 + r, ny - 1), i = imin(ti * 16 + r, nx - 1);
+    const int K = pass == 0 || pass == 3 ? nx : ny, Kw = (K + 15) / 16 * 4;
+    const int q0 = imin(w * Kw, K), q1 = imin(q0 + Kw, K);
+    mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+    if (q0 < q1) {
+        if (pass == 0)
+            mfma_tile<8>(q0, q1, [&](int q) { return (double)in[j * nx + q]; }, [&](int q) { return Vx[q * nx + i]; },
+                         acc);
+        else if (pass == 1)
+            mfma_tile<8>(q0, q1, [&](int q) { return Vy[q * ny + j]; }, [&](int q) { return (double)in[q * nx + i]; },
+                         acc);
+        else if (pass == 2)
+            mfma_tile<8>(q0, q1, [&](int q) { return Vy[j * ny + q]; }, [&](int q) { return (double)in[q * nx + i]; },
+                         acc);
         else
-            for (int q = 0; q < nx; ++q) acc += Vx[q * nx + i] * a[q];
-        dst[(int64_t)j0 * nx + e] = (Tout)acc;
+            mfma_tile<8>(q0, q1, [&](int q) { return (double)in[j * nx + q]; }, [&](int q) { return Vx[i * nx + q]; },
+                         acc);
     }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) lds[w * 256 + (4 * v + (lane >> 4)) * 16 + r] = acc[v];
+    __syncthreads();
+    const int e = threadIdx.x, jo = tj * 16 + (e >> 4), io = ti * 16 + (e & 15);
+    if (jo >= ny || io >= nx) return;
+    double val = ((lds[e] + lds[256 + e]) + lds[512 + e]) + lds[768 + e];
+    if (pass == 1) {
+        const double lam = lx[io] + ly[jo];
+        val = lam > eps ? val / (s * lam) : 0.0;
+    }
+    out[jo * nx + io] = (Tout)val;
 }
 
-// columns [blk*C, blk*C + C) of pass 1, in place on t; lds: 2*ny*C doubles, then the staged basis
-// (fdm2_cols_lds)
-__device__ __forceinline__ void fdm2_cols_body(double* lds, int nx, int ny, int blk, double* t, const double* Vy,
-                                               const double* lx, const double* ly, double s, double eps) {
-    const int C = fdm2_cols_per(ny);
-    const int i0 = blk * C;
-    const int nc = min(C, nx - i0);
-    const int P = ny * nc;
-    double* a = lds;
-    double* b = lds + ny * C;
-    // the columns (a[j*C+ci]; columns past the grid's last hold a copy of
-    // its value, never read) and the basis in one round of loads
-    const bool sv = ny * ny <= kFdmVStage;
-    lds_fill2<1, 16>(
-        a, ny * C,
-        [&](int e) {
-            const int j = e / C, ci = e - j * C;
-            return t[(int64_t)j * nx + i0 + imin(ci, nc - 1)];
-        },
-        lds + 2 * ny * C, sv ? ny * ny : 0, [&](int e) { return Vy[e]; });
-    if (sv) Vy = lds + 2 * ny * C;
-    __syncthreads();
-    for (int e = threadIdx.x; e < P; e += blockDim.x) {
-        int j = e / nc, ci = e - j * nc;
-        double acc = 0.0;
-        for (int q = 0; q < ny; ++q) acc += Vy[q * ny + j] * a[q * C + ci];
-        double lam = lx[i0 + ci] + ly[j];
-        b[j * C + ci] = lam > eps ? acc / (s * lam) : 0.0;
+// The whole solve of a level of at most kFdm2One x kFdm2One cells in one
+// workgroup of kFdm2Threads: both bases and two planes in LDS as N x N arrays
+// (N the next of 16, 32, 64; zero past the level, so no product needs a bound
+// and every LDS offset is a constant), rows padded by two entries, so the 16
+// rows that a wave reads together fall into different banks. One 16 x 16 tile
+// per wave and product. (64 x 64 with bounds and row lengths at run time: 18 us.)
+constexpr int kFdm2One = 64, kFdm2Threads = 1024;
+__host__ __device__ inline bool fdm2_one(int nx, int ny) { return nx <= kFdm2One && ny <= kFdm2One; }
+__host__ __device__ inline int fdm2_one_n(int nx, int ny) {
+    const int n = nx > ny ? nx : ny;
+    return n <= 16 ? 16 : n <= 32 ? 32 : 64;
+}
+__host__ __device__ inline size_t fdm2_one_lds(int nx, int ny) {
+    const int N = fdm2_one_n(nx, ny);
+    return (size_t)4 * N * (N + 2) * sizeof(double);
+}
+// dst = src where a's operand is a row (AT: a column) of A and B's a column (BT: a row)
+template <int N, bool AT, bool BT>
+__device__ __forceinline__ mfma_d4 fdm2_lds_tile(const double* A, const double* B, int j0, int i0) {
+    constexpr int P = N + 2;
+    const int lane = threadIdx.x & 63, r = lane & 15, k = lane >> 4;
+    const double* a = A + (AT ? k * P + j0 + r : (j0 + r) * P + k);
+    const double* b = B + (BT ? (i0 + r) * P + k : k * P + i0 + r);
+    mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < N; q += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[AT ? q * P : q], b[BT ? q : q * P], acc, 0, 0, 0);
+    return acc;
+}
+template <int N, typename Tin, typename Tout>
+__device__ __forceinline__ void fdm2_one_n_body(double* lds, int nx, int ny, const Tin* in, Tout* out,
+                                                const double* Vx, const double* Vy, const double* lx,
+                                                const double* ly, double s, double eps) {
+    constexpr int P = N + 2, U = (N * N + kFdm2Threads - 1) / kFdm2Threads;
+    double *a = lds, *b = a + N * P, *vx = b + N * P, *vy = vx + N * P;
+    {   // the plane and the bases, all loads in flight together
+        double v0[U], v1[U], v2[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = threadIdx.x + u * kFdm2Threads, q = e / N, i = e % N;
+            const bool ox = i < nx, oy = q < ny;
+            v0[u] = (double)in[ox && oy ? q * nx + i : 0];
+            v1[u] = Vx[ox && q < nx ? q * nx + i : 0];
+            v2[u] = Vy[i < ny && oy ? q * ny + i : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = threadIdx.x + u * kFdm2Threads, q = e / N, i = e % N;
+            if (q >= N) continue;
+            const bool ox = i < nx, oy = q < ny;
+            a[q * P + i] = ox && oy ? v0[u] : 0.0;
+            vx[q * P + i] = ox && q < nx ? v1[u] : 0.0;
+            vy[q * P + i] = i < ny && oy ? v2[u] : 0.0;
+        }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < P; e += blockDim.x) {
-        int j = e / nc, ci = e - j * nc;
-        double acc = 0.0;
-        for (int k = 0; k < ny; ++k) acc += Vy[j * ny + k] * b[k * C + ci];
-        t[(int64_t)j * nx + i0 + ci] = acc;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i0 = w % (N / 16) * 16, j0 = w / (N / 16) * 16;
+    const int io = i0 + (lane & 15), jo = j0 + (lane >> 4);  // the lane's outputs: rows jo + 4 v
+    const bool on = w < (N / 16) * (N / 16);
+    if (on) {
+        const mfma_d4 c = fdm2_lds_tile<N, false, false>(a, vx, j0, i0);  // R Vx
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b[(jo + 4 * v) * P + io] = c[v];
+    }
+    __syncthreads();
+    if (on) {
+        const mfma_d4 c = fdm2_lds_tile<N, true, false>(vy, b, j0, i0);  // Vy^T (R Vx), scaled
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int jv = jo + 4 * v;
+            const double lam = io < nx && jv < ny ? lx[io] + ly[jv] : 0.0;
+            a[jv * P + io] = lam > eps ? c[v] / (s * lam) : 0.0;
+        }
+    }
+    __syncthreads();
+    if (on) {
+        const mfma_d4 c = fdm2_lds_tile<N, false, false>(vy, a, j0, i0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b[(jo + 4 * v) * P + io] = c[v];
+    }
+    __syncthreads();
+    if (on) {
+        const mfma_d4 c = fdm2_lds_tile<N, false, true>(b, vx, j0, i0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (io < nx && jo + 4 * v < ny) out[(jo + 4 * v) * nx + io] = (Tout)c[v];
+    }
+}
+template <typename Tin, typename Tout>
+__device__ __forceinline__ void fdm2_one_body(double* lds, int nx, int ny, const Tin* in, Tout* out, const double* Vx,
+                                              const double* Vy, const double* lx, const double* ly, double s,
+                                              double eps) {
+    switch (fdm2_one_n(nx, ny)) {
+        case 16: fdm2_one_n_body<16>(lds, nx, ny, in, out, Vx, Vy, lx, ly, s, eps); break;
+        case 32: fdm2_one_n_body<32>(lds, nx, ny, in, out, Vx, Vy, lx, ly, s, eps); break;
+        default: fdm2_one_n_body<64>(lds, nx, ny, in, out, Vx, Vy, lx, ly, s, eps); break;
     }
 }
 
