@@ -498,7 +498,7 @@ pano_status hgrid_layout(Ctx* c, HGrid& g, int64_t base, bool proj) {
     g.bytes = off - base;
     PANO_CHECK(axis_basis(c, C.w, C.bc & 1, (C.bc >> 1) & 1, (double**)&g.Vx, (double**)&g.lx));
     PANO_CHECK(axis_basis(c, C.h, (C.bc >> 2) & 1, (C.bc >> 3) & 1, (double**)&g.Vy, (double**)&g.ly));
-    if (C.d > 1) {
+    if (D.d > 1) {  // also where the coarsest level is a single plane
         PANO_CHECK(axis_basis(c, C.d, (C.bc >> 4) & 1, (C.bc >> 5) & 1, (double**)&g.Vz, (double**)&g.lz));
     } else {
         g.Vz = nullptr;

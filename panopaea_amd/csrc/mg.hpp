@@ -22,9 +22,10 @@ struct MG {
     int coarse_n[3] = {1, 1, 1};                         // coarsest extents x, y, z
     bool tb = true;  // 3D f32 levels: pre/post-smoothing as one pass each (PANO_MG_FUSED=0 turns it off)
     bool fdm_split = false;  // 3D coarsest level: passes split over many workgroups (PANO_FDM_SPLIT=0: off)
-    // f32 one-pass levels above the coarsest: the prolongation runs inside
-    // the post-smoothing (PANO_MG_PRO=0: off), which then reads the
-    // pre-smoothed z from w[l] (the down leg's z) while it writes z.
+    // levels above the coarsest that smooth in one pass or run their legs as
+    // one launch each: the prolongation runs inside the post-smoothing
+    // (PANO_MG_PRO=0: off), which then reads the pre-smoothed z from w[l]
+    // (the down leg's z) while it writes z.
     bool pro = false;
     T* w[16] = {};
 };
@@ -39,6 +40,9 @@ pano_status mg_check(const Dims& D, int levels);
 
 template <typename T>
 pano_status mg_setup(Ctx* c, const Dims& D, int levels, int nu, double dt, MG<T>* m);
+
+// Workgroups of a level's up leg (two z.r partials each).
+int mg_leg_blocks(const Dims& D);
 
 // z0 = M r0 (one V-cycle from zero), both in red-black layout at level 0.
 // Every kernel returns at once when st->done is set.

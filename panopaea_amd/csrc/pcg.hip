@@ -158,12 +158,14 @@ struct Solver {
 };
 
 // Entries of each partial-sum array: one per flat block, two per tile (the
-// red-black V-cycle's two sweeps), and one per tile of the fused step's
+// red-black V-cycle's two sweeps; at least two per workgroup of its up leg),
+// and one per tile of the fused step's
 // divergence (its max|b| partials).
 static int solver_partials(const Dims& D, bool rb) {
     const int nflat = (int)blocks_for((int64_t)D.d * D.h * D.w, kFlatPer);
     const int ntile = (rb ? grid3_rb(D) : grid3(D.w, D.h, D.d)).nb;
     int np = nflat > 2 * ntile ? nflat : 2 * ntile;
+    if (rb && 2 * mg_leg_blocks(D) > np) np = 2 * mg_leg_blocks(D);
     const Grid3 Gd = grid3_run(D.w, D.h, D.d, D.d > 1 ? kPlaneRun<3> : 1);
     return Gd.nb > np ? Gd.nb : np;
 }
