@@ -31,13 +31,14 @@
 
 namespace pano {
 
-template <int TX, int TY>
+// DENS: the density is advected too (without it, it is not staged either).
+template <int TX, int TY, bool DENS = true>
 struct AdvShape {
     static constexpr int NT = TX * TY;
     static constexpr int RW = TX + 2, RH = TY + 2;  // cell box (tile + 1 on each side)
     static constexpr int XW = TX + 3;                // x faces per box row (x0-1 .. x0+TX+1)
     static constexpr int YH = TY + 3;                // y-face rows (y0-1 .. y0+TY+1)
-    static constexpr int O_RHO = 0, O_VZ = RH * RW, O_VX = 2 * RH * RW, O_VY = 2 * RH * RW + RH * XW;
+    static constexpr int O_RHO = 0, O_VZ = DENS ? RH * RW : 0, O_VX = O_VZ + RH * RW, O_VY = O_VX + RH * XW;
     static constexpr int SLOT = O_VY + YH * RW;
     static constexpr int SLOTS = 4;
     static constexpr int LDS_FLOATS = SLOTS * SLOT;
@@ -45,24 +46,26 @@ struct AdvShape {
     static constexpr int KC = (RH * RW + NT - 1) / NT, KX = (RH * XW + NT - 1) / NT, KY = (YH * RW + NT - 1) / NT;
 };
 
-// Workgroup chunks: tiles of TX x TY cells by chunks of zc planes.
+// Workgroup chunks: tiles of TX x TY cells by chunks of zc planes, halved down
+// to 2 while the launch has fewer than `want` workgroups.
 struct AdvGrid {
     int gx, gy, zc, nch, nb;
 };
 template <int TX, int TY>
-inline AdvGrid adv_grid(const Dims& D, int zc) {
+inline AdvGrid adv_grid(const Dims& D, int zc, int want = 0) {
     AdvGrid g;
     g.gx = (D.w + TX - 1) / TX;
     g.gy = (D.h + TY - 1) / TY;
+    while (zc > 2 && (int64_t)g.gx * g.gy * ((D.d + zc - 1) / zc) < want) zc /= 2;
     g.zc = zc < D.d ? zc : D.d;
     g.nch = (D.d + g.zc - 1) / g.zc;
     g.nb = g.gx * g.gy * g.nch;
     return g;
 }
 
-template <int TX, int TY>
+template <int TX, int TY, bool DENS = true>
 struct AdvThread {
-    using S = AdvShape<TX, TY>;
+    using S = AdvShape<TX, TY, DENS>;
     static constexpr int RW = S::RW, RH = S::RH, XW = S::XW, YH = S::YH, NT = S::NT, KC = S::KC, KX = S::KX,
                          KY = S::KY, SLOT = S::SLOT;
 
@@ -151,7 +154,7 @@ struct AdvThread {
         const float* yp = v.y + pcl * (D.h + 1) * D.w;
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
-            p_rho[k] = (cell_p && vc[k]) ? ldx(rp, gc[k]) : 0.0f;
+            if constexpr (DENS) p_rho[k] = (cell_p && vc[k]) ? ldx(rp, gc[k]) : 0.0f;
             p_vz[k] = (face_p && vc[k]) ? ldx(zp, gc[k]) : 0.0f;
         }
 #pragma unroll
@@ -167,9 +170,11 @@ struct AdvThread {
 #pragma unroll
         for (int k = 0; k < KC; ++k) {
             if (!vcx[k]) continue;
-            float r = p_rho[k];
-            if (Sph.on && cell_p && vc[k] && in_sphere(Sph, D, p, cy_[k], cx_[k])) r = 1.0f;
-            s[S::O_RHO + ec[k]] = r;
+            if constexpr (DENS) {
+                float r = p_rho[k];
+                if (Sph.on && cell_p && vc[k] && in_sphere(Sph, D, p, cy_[k], cx_[k])) r = 1.0f;
+                s[S::O_RHO + ec[k]] = r;
+            }
             s[S::O_VZ + ec[k]] = p_vz[k];
         }
 #pragma unroll
@@ -315,7 +320,7 @@ struct AdvThread {
             for (int j = 0; j < 8; ++j) g[j] = ldx(v.z, fz_idx(D, gz[j >> 2], gy[(j >> 1) & 1], gx[j & 1]));
         }
         float val = trilerp(g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7], sw, tw, uw);
-        if (buoy_c != zero) {
+        if (DENS && buoy_c != zero) {
             const float rlo = zf > 0 ? l_rho(zf - 1, y, x) : zero;
             const float rhi = zf < D.d ? l_rho(zf, y, x) : zero;
             const bool open_face = (zf > 0 && zf < D.d) || (zf == 0 && (D.bc & 16)) || (zf == D.d && (D.bc & 32));
@@ -339,11 +344,12 @@ struct AdvThread {
     }
     __host__ __device__ __forceinline__ void outputs(int z) {
         if (!act) return;
-        const float c = cell_value(z);
+        float c = 0.0f;
+        if constexpr (DENS) c = cell_value(z);
         const float fx = xface_value(z, x);
         const float fy = yface_value(z, y);
         const float fz = zface_value(z, z);
-        stx(rho_o, cell_index(D, z, y, x), c);
+        if constexpr (DENS) stx(rho_o, cell_index(D, z, y, x), c);
         stx(vo.x, fx_idx(D, z, y, x), fx);
         stx(vo.y, fy_idx(D, z, y, x), fy);
         stx(vo.z, fz_idx(D, z, y, x), fz);

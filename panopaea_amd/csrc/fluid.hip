@@ -6,6 +6,7 @@
 // workgroup order is remapped so each XCD sweeps a contiguous slab.
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "adv_fused.hpp"
 #include "fluid_device.hpp"
@@ -73,19 +74,21 @@ __global__ __launch_bounds__(256) void k_advect_fz(Dims D, Grid3 G, T* dst, cons
         if (z0 + k <= D.d) stx(dst, fz_idx(D, z0 + k, y, x), out[k]);
 }
 
-// The step's advection of a 3D f32 grid in one pass: density and the three
-// face components, a TX x TY column over a chunk of planes per workgroup,
-// gathers from a ring of staged planes in LDS (AdvThread). At most 128 VGPRs,
-// so two workgroups share a CU (measured: 333 us at 256^3 against 477 us at
-// the compiler's own 146 VGPRs, and 488 us for the four per-component kernels).
-constexpr int kAdvTX = 64, kAdvTY = 8, kAdvZC = 16;
-__global__ __launch_bounds__(kAdvTX * kAdvTY) __attribute__((amdgpu_waves_per_eu(4))) void k_advect_fused(Dims D, AdvGrid g, Faces<const float> v,
-                                                                  const float* rho, Faces<float> vo, float* rho_o,
-                                                                  Sphere S, float dt, float buoy_c) {
-    __shared__ float lds[AdvShape<kAdvTX, kAdvTY>::LDS_FLOATS];
+// Advection of a 3D f32 grid in one pass: the three face components, in the
+// step (DENS) with the density, a TX x TY column over a chunk of planes per
+// workgroup, gathers from a ring of staged planes in LDS (AdvThread). At most
+// 128 VGPRs, so two workgroups share a CU (measured: 333 us at 256^3 against
+// 477 us at the compiler's own 146 VGPRs, and 488 us for the four
+// per-component kernels). The density alone stays with its kernel (125x131x193
+// 30 us, 29 to 34 from staged planes).
+template <int TX, int TY, bool DENS>
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(4))) void k_advect_fused(
+    Dims D, AdvGrid g, Faces<const float> v, const float* rho, Faces<float> vo, float* rho_o, Sphere S, float dt,
+    float buoy_c) {
+    __shared__ float lds[AdvShape<TX, TY, DENS>::LDS_FLOATS];
     const int L = xcd_remap(blockIdx.x, g.nb);
     const int bx = L % g.gx, q = L / g.gx, by = q % g.gy, bz = q / g.gy;
-    AdvThread<kAdvTX, kAdvTY> th;
+    AdvThread<TX, TY, DENS> th;
     th.init(lds, D, bx, by, bz, g.zc, v, rho, vo, rho_o, S, dt, buoy_c, threadIdx.x);
     th.prologue();
     __syncthreads();
@@ -223,6 +226,30 @@ pano_status launch_advect(Ctx* c, const Dims& D, T* dst, const T* src, double dt
     return PANO_OK;
 }
 
+bool advect_fused_on(const Dims& D) {
+    const char* e = getenv("PANO_ADV_FUSED");
+    return D.d > 1 && !(e && e[0] == '0');
+}
+
+// The one-pass advection's launch. Tiles of 32 x 16 cells (256^3 faces 211 us
+// against 233 as 64 x 8: less halo), or of 64 x 8 where those cover the plane
+// with fewer cells outside it (40 x 40 planes: 12.5 us against 16.3). Chunks of
+// 16 planes, shorter while there are fewer than 512 workgroups (64^3 step: 61 us
+// with 32 workgroups, 14 with 256).
+template <bool DENS>
+static void launch_fused(Ctx* c, const char* name, double bytes, const Dims& D, float* rho_out, const float* rho_in,
+                         float* vel_out, const float* vel_in, double dt, double buoy_c, const double* src_sphere) {
+    auto go = [&](auto tx, auto ty) {
+        constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
+        const AdvGrid g = adv_grid<TX, TY>(D, 16, 512);
+        klaunch(c, name, bytes, k_advect_fused<TX, TY, DENS>, dim3(g.nb), dim3(TX * TY), D, g, split_faces(D, vel_in),
+                rho_in, split_faces(D, vel_out), rho_out, make_sphere(src_sphere), (float)dt, (float)buoy_c);
+    };
+    const AdvGrid a = adv_grid<32, 16>(D, 16), b = adv_grid<64, 8>(D, 16);  // same cells per tile
+    if (b.nb < a.nb) go(std::integral_constant<int, 64>{}, std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
+}
+
 template <typename T>
 pano_status launch_advect_mac(Ctx* c, const Dims& D, T* dst, const T* src, double dt, const T* vel,
                               double buoy_c, const T* rho, const double* src_sphere) {
@@ -232,6 +259,15 @@ pano_status launch_advect_mac(Ctx* c, const Dims& D, T* dst, const T* src, doubl
     Sphere S = make_sphere(src_sphere);
     const int nz = D.d > 1 ? kAdvectRun<3> : 1;
     Grid3 Gx = grid3_run(D.w + 1, D.h, D.d, nz), Gy = grid3_run(D.w, D.h + 1, D.d, nz);
+    if constexpr (sizeof(T) == 4) {
+        // the velocity advected by itself: all three components in one pass
+        if (src == vel && buoy_c == 0.0 && advect_fused_on(D)) {
+            launch_fused<false>(c, "advect_mac", 6.0 * D.d * D.h * D.w * sizeof(T), D, (float*)nullptr,
+                                (const float*)nullptr, dst, vel, dt, 0.0, src_sphere);
+            PANO_HIP(hipGetLastError());
+            return PANO_OK;
+        }
+    }
     if (D.d > 1) {
         Grid3 Gz = grid3_run(D.w, D.h, D.d + 1, nz);
         LAUNCH3((k_advect_fx<T, 3>), Gx, D, Gx, o.x, q.x, (T)dt, v);
@@ -244,19 +280,11 @@ pano_status launch_advect_mac(Ctx* c, const Dims& D, T* dst, const T* src, doubl
     return PANO_OK;
 }
 
-bool advect_fused_on(const Dims& D) {
-    const char* e = getenv("PANO_ADV_FUSED");
-    return D.d > 1 && !(e && e[0] == '0');
-}
-
 pano_status launch_advect_fused(Ctx* c, const Dims& D, float* rho_out, const float* rho_in, float* vel_out,
                                 const float* vel_in, double dt, double buoy_c, const double* src_sphere) {
-    const AdvGrid g = adv_grid<kAdvTX, kAdvTY>(D, kAdvZC);
-    const double cells = (double)D.d * D.h * D.w * sizeof(float);
     // read rho and the three components once, write them once
-    klaunch(c, "advect_fused", 8.0 * cells, k_advect_fused, dim3(g.nb), dim3(kAdvTX * kAdvTY), D, g,
-            split_faces(D, vel_in), rho_in, split_faces(D, vel_out), rho_out, make_sphere(src_sphere), (float)dt,
-            (float)buoy_c);
+    launch_fused<true>(c, "advect_fused", 8.0 * D.d * D.h * D.w * sizeof(float), D, rho_out, rho_in, vel_out, vel_in,
+                       dt, buoy_c, src_sphere);
     PANO_HIP(hipGetLastError());
     return PANO_OK;
 }
