@@ -123,11 +123,11 @@ __global__ __launch_bounds__(256) void kb_project(BTab T, char* A) {
 
 // One workgroup per grid: reduces the grid's partials of the launch `tab`
 // (blocks [start, start + G.nb)) and updates its state.
-__global__ __launch_bounds__(1024) void kb_finalize(int op, BTab T, const double* part0, const double* part1,
+__global__ __launch_bounds__(256) void kb_finalize(int op, BTab T, const double* part0, const double* part1,
                                                     SolverState* st, const SolveCfg* cfg, int use_max) {
     const BEntry& E = T.e[blockIdx.x];
-    finalize_range(op, part0 + E.start, part1 ? part1 + E.start : nullptr, E.G.nb, &st[E.sidx], cfg[E.sidx],
-                   use_max);
+    finalize_range<256>(op, part0 + E.start, part1 ? part1 + E.start : nullptr, E.G.nb, &st[E.sidx], cfg[E.sidx],
+                        use_max);
     if (op == FIN_STATS && threadIdx.x == 0 && !cfg[E.sidx].remove_mean) st[E.sidx].mean = 0.0;
 }
 
@@ -918,7 +918,7 @@ pano_status BatchCore::build(const std::vector<HGrid>& grids, const std::vector<
 
 void BatchCore::fin(int op, const double* p0, const double* p1, const Table& t, int use_max) {
     if (t.h.empty()) return;
-    hipLaunchKernelGGL(kb_finalize, dim3((unsigned)t.h.size()), dim3(1024), 0, c->stream, op, t.view(), p0, p1,
+    hipLaunchKernelGGL(kb_finalize, dim3((unsigned)t.h.size()), dim3(256), 0, c->stream, op, t.view(), p0, p1,
                        states, (const SolveCfg*)cfgs, use_max);
 }
 

@@ -145,74 +145,96 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
 }
 
 // ---- wavefront / block reductions (64-wide wavefronts) -----------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// v of lane ^ O, for O = 32, 16, 8, 4, 2, 1, without LDS (a shuffle is a
+// ds_bpermute per word and step, six dependent LDS round trips per wave).
+// O = 32 and 16 use the row swaps of two copies of v: one result holds the
+// even halves (rows) twice, the other the odd ones, and the operation of the
+// two is that of v and its partner in either order.
+template <int O>
+__device__ __forceinline__ int lane_xor(int v) {
+    if constexpr (O == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);  // row_ror:8
+    else if constexpr (O == 4) {  // row_shl:4 into the even quads, row_shr:4 into the odd ones
+        const int lo = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xF, 0x5, false);
+        return __builtin_amdgcn_update_dpp(lo, v, 0x114, 0xF, 0xA, false);
+    } else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
+    else return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
+}
+// a and b: v and v of lane ^ O, in an order that is the same for both lanes
+template <int O>
+__device__ __forceinline__ void lane_pair(double v, double& a, double& b) {
+    const long long w = __double_as_longlong(v);
+    const int lo = (int)w, hi = (int)(w >> 32);
+    if constexpr (O >= 16) {
+        auto swap = [](int x) {
+            if constexpr (O == 32) return __builtin_amdgcn_permlane32_swap(x, x, false, false);
+            else return __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        };
+        const auto l = swap(lo), h = swap(hi);
+        a = __longlong_as_double(((long long)h[0] << 32) | (unsigned)l[0]);
+        b = __longlong_as_double(((long long)h[1] << 32) | (unsigned)l[1]);
+    } else {
+        a = v;
+        b = __longlong_as_double(((long long)lane_xor<O>(hi) << 32) | (unsigned)lane_xor<O>(lo));
+    }
 }
 // max that keeps a NaN from either side (fmax would drop it): the norms built
 // from it are NaN as soon as one term is, so the solver's NaN tests see it.
 __device__ __forceinline__ double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = nan_max(v, __shfl_xor(v, o, 64));
-    return v;
+template <int O, bool MAX>
+__device__ __forceinline__ double lane_step(double v) {
+    double a, b;
+    lane_pair<O>(v, a, b);
+    return MAX ? nan_max(a, b) : a + b;
 }
-// Block of blockDim.x*blockDim.y*blockDim.z threads (a multiple of 64, <= 1024).
-// Fixed butterfly + fixed LDS order: deterministic. Result valid in thread 0.
-__device__ __forceinline__ double block_sum(double v) {
-    __shared__ double red_s[16];
-    int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-    int nthr = blockDim.x * blockDim.y * blockDim.z;
-    v = wave_sum(v);
+template <bool MAX>
+__device__ __forceinline__ double wave_reduce(double v) {
+    v = lane_step<32, MAX>(v);
+    v = lane_step<16, MAX>(v);
+    v = lane_step<8, MAX>(v);
+    v = lane_step<4, MAX>(v);
+    v = lane_step<2, MAX>(v);
+    return lane_step<1, MAX>(v);
+}
+__device__ __forceinline__ double wave_sum(double v) { return wave_reduce<false>(v); }
+__device__ __forceinline__ double wave_max(double v) { return wave_reduce<true>(v); }
+
+// Block reductions over NT threads (whole waves) from the wave results: fixed
+// butterfly + the waves in order, deterministic. `wave` and `first` are the
+// caller's wave and whether it is the wave's first lane; the result is valid
+// in the first lane of wave 0. All of the waves' results are read before they
+// are combined.
+template <int NT, bool MAX>
+__device__ __forceinline__ double block_reduce(double v, int wave, bool first, double* red) {
+    v = wave_reduce<MAX>(v);
     __syncthreads();
-    if ((tid & 63) == 0) red_s[tid >> 6] = v;
+    if (first) red[wave] = v;
     __syncthreads();
     double s = 0.0;
-    if (tid == 0)
-        for (int i = 0; i < (nthr >> 6); ++i) s += red_s[i];
+    if (first && wave == 0) {
+        double r[NT / 64];
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) r[i] = red[i];
+#pragma unroll
+        for (int i = 0; i < NT / 64; ++i) s = MAX ? nan_max(s, r[i]) : s + r[i];
+    }
     return s;
+}
+// Workgroups of kBlock threads in any two-dimensional shape.
+__device__ __forceinline__ double block_sum(double v) {
+    __shared__ double red_s[kBlock / 64];
+    const int tid = threadIdx.x + blockDim.x * threadIdx.y;
+    return block_reduce<kBlock, false>(v, tid >> 6, (tid & 63) == 0, red_s);
 }
 __device__ __forceinline__ double block_max(double v) {
-    __shared__ double redm_s[16];
-    int tid = threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z);
-    int nthr = blockDim.x * blockDim.y * blockDim.z;
-    v = wave_max(v);
-    __syncthreads();
-    if ((tid & 63) == 0) redm_s[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (tid == 0)
-        for (int i = 0; i < (nthr >> 6); ++i) s = nan_max(s, redm_s[i]);
-    return s;
+    __shared__ double redm_s[kBlock / 64];
+    const int tid = threadIdx.x + blockDim.x * threadIdx.y;
+    return block_reduce<kBlock, true>(v, tid >> 6, (tid & 63) == 0, redm_s);
 }
-
-// The same two reductions for a one-dimensional workgroup (blockDim.y =
-// blockDim.z = 1): identical arithmetic, without reading the workgroup's
-// other extents (a memory load in the middle of the kernel).
-__device__ __forceinline__ double block_sum_x(double v) {
-    __shared__ double redx_s[16];
-    const int tid = threadIdx.x;
-    v = wave_sum(v);
-    __syncthreads();
-    if ((tid & 63) == 0) redx_s[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (tid == 0)
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += redx_s[i];
-    return s;
-}
-__device__ __forceinline__ double block_max_x(double v) {
-    __shared__ double redmx_s[16];
-    const int tid = threadIdx.x;
-    v = wave_max(v);
-    __syncthreads();
-    if ((tid & 63) == 0) redmx_s[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (tid == 0)
-        for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s = nan_max(s, redmx_s[i]);
-    return s;
+// One-dimensional workgroups of NT threads.
+template <int NT, bool MAX>
+__device__ __forceinline__ double block_reduce_x(double v) {
+    __shared__ double redx_s[NT / 64];
+    return block_reduce<NT, MAX>(v, threadIdx.x >> 6, (threadIdx.x & 63) == 0, redx_s);
 }
 
 // Two sums at once over a one-dimensional workgroup of NT threads: each with

@@ -23,9 +23,17 @@
 
 namespace pano {
 
-__global__ __launch_bounds__(1024) void k_finalize(int op, const double* part, const double* part1, int np,
-                                                   SolverState* st, SolveCfg cfg, int use_max) {
-    finalize_range(op, part, part1, np, st, cfg, use_max);
+template <int NT>
+__global__ __launch_bounds__(NT) void k_finalize(int op, const double* part, const double* part1, int np,
+                                                 SolverState* st, SolveCfg cfg, int use_max) {
+    finalize_range<NT>(op, part, part1, np, st, cfg, use_max);
+}
+static void launch_finalize(hipStream_t s, int op, const double* part, const double* part1, int np, SolverState* st,
+                            const SolveCfg& cfg, int use_max) {
+    if (np <= kFinSmall)
+        hipLaunchKernelGGL(k_finalize<256>, dim3(1), dim3(256), 0, s, op, part, part1, np, st, cfg, use_max);
+    else
+        hipLaunchKernelGGL(k_finalize<1024>, dim3(1), dim3(1024), 0, s, op, part, part1, np, st, cfg, use_max);
 }
 
 // q = A p with partial p.q ; natural layout, optional 2D obstacle mask.
@@ -240,8 +248,7 @@ static pano_status solver_setup(Ctx* c, const Dims& D, const pano_pcg_params* P,
 // part1 (optional) holds a second set of np partials added element by element.
 template <typename T>
 static void fin(Solver<T>* S, int op, double* part, int np, int use_max, const double* part1 = nullptr) {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, S->c->stream, op, (const double*)part, part1, np, S->st,
-                       S->cfg, use_max);
+    launch_finalize(S->c->stream, op, part, part1, np, S->st, S->cfg, use_max);
     if (op == FIN_RNORM) S->c->timer.checks += 1;
 }
 
@@ -776,15 +783,11 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
     hipLaunchKernelGGL((k_zero_stats<double>), dim3(S.nflat), dim3(kBlock), 0, s, n, xx, (const double*)bb, S.part0,
                        part);
     if (cfg2.remove_mean) {
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, s, (int)FIN_STATS, (const double*)S.part0,
-                           (const double*)nullptr, S.nflat,
-                           st2, cfg2, 0);
+        launch_finalize(s, FIN_STATS, S.part0, nullptr, S.nflat, st2, cfg2, 0);
         hipLaunchKernelGGL((k_sub_mean<double>), dim3(S.nflat), dim3(kBlock), 0, s, n, bb, (const SolverState*)st2,
                            part);
     }
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, s, (int)FIN_THRESH, (const double*)part,
-                       (const double*)nullptr, S.nflat, st2,
-                       cfg2, 1);
+    launch_finalize(s, FIN_THRESH, part, nullptr, S.nflat, st2, cfg2, 1);
     SolverState* hs = c->host_state;
     const std::string key = hint_key(D, &ip, sizeof(float));
     int outer = 0, inner_total = 0;
@@ -796,8 +799,7 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
         else
             hipLaunchKernelGGL(k_resid64_rb<2>, dim3(Gr.nb), dim3(kTX, kTY), 0, s, D, Gr, S.r, (const double*)xx,
                                (const double*)bb, M->inner.dt, part);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, s, (int)FIN_RNORM, (const double*)part,
-                           (const double*)nullptr, Gr.nb, st2, cfg2, 1);
+        launch_finalize(s, FIN_RNORM, part, nullptr, Gr.nb, st2, cfg2, 1);
         PANO_HIP(hipMemcpyAsync(&hs[1], st2, sizeof(SolverState), hipMemcpyDeviceToHost, s));
         PANO_HIP(hipStreamSynchronize(s));
         if (hs[1].done) break;

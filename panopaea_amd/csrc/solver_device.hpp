@@ -25,10 +25,14 @@ struct SolveCfg {
 
 // Reduces the FP64 partials part0[0..np) (+ part1[0..np) when part1 is not
 // null) in a fixed order and applies `op` to the solver state. Run by one
-// one-dimensional workgroup (all threads). The state is read once, at the
+// one-dimensional workgroup of NT threads (all of them), 256 up to kFinSmall partials:
+// a few thousand partials are one round of loads for 256 threads, whose four
+// waves are started and combined faster than sixteen. The state is read once, at the
 // start, and the done test comes at the end, after the reduction (the
 // partials' loads no longer wait for it): a finished solve (done) changes
 // nothing; its partials are read and left unused.
+constexpr int kFinSmall = 2048;  // partials up to which 256 threads reduce
+template <int NT>
 __device__ __forceinline__ void finalize_range(int op, const double* part0, const double* part1, int np,
                                                SolverState* st, const SolveCfg& cfg, int use_max) {
     const SolverState s0 = *st;
@@ -36,31 +40,31 @@ __device__ __forceinline__ void finalize_range(int op, const double* part0, cons
     // loads are unconditional (indices past the end read the last partial and
     // count as 0), so all of a thread's loads are in flight together
     double a8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int stride = blockDim.x * 8;
+    const int stride = NT * 8;
     for (int base = threadIdx.x; base < np; base += stride) {
         double v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const int i = base + u * blockDim.x;
+            const int i = base + u * NT;
             v[u] = part0[i < np ? i : np - 1];
         }
         if (part1) {
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int i = base + u * blockDim.x;
+                const int i = base + u * NT;
                 v[u] += part1[i < np ? i : np - 1];
             }
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const double w = base + u * (int)blockDim.x < np ? v[u] : 0.0;
+            const double w = base + u * NT < np ? v[u] : 0.0;
             a8[u] = use_max ? absmax_acc(a8[u], w) : a8[u] + w;
         }
     }
     double acc = 0.0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc = use_max ? absmax_acc(acc, a8[u]) : acc + a8[u];
-    double tot = use_max ? block_max_x(acc) : block_sum_x(acc);  // one-dimensional workgroup
+    double tot = use_max ? block_reduce_x<NT, true>(acc) : block_reduce_x<NT, false>(acc);
     if (threadIdx.x != 0) return;
     if (op >= FIN_SIGMA0 && s0.done) return;
     switch (op) {
