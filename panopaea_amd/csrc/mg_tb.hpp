@@ -351,8 +351,8 @@ struct TbThread {
         const float* p1 = p0 + n2;
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
-            xpf[0][k] = p0[goff[k]];
-            xpf[1][k] = p1[goff[k]];
+            if constexpr (!(PRO && CF == 0)) xpf[0][k] = p0[goff[k]];
+            if constexpr (!(PRO && CF == 1)) xpf[1][k] = p1[goff[k]];
         }
     }
     __host__ __device__ __forceinline__ bool load_b(int z, float (&v)[2][KP]) const {
@@ -381,17 +381,20 @@ struct TbThread {
         for (int k = 0; k < KP; ++k) {
             if ((k % KC) * NT + tid < CPOS) {
                 const bool ok = xok && ind[k];
-                float v0 = xpf[0][k], v1 = xpf[1][k];
                 if constexpr (PRO) {
-                    const float pl = wz0 * q0[0][k] + wz1 * q1[0][k];  // cell x = 2m
-                    const float pr = wz0 * q0[1][k] + wz1 * q1[1][k];  // cell x = 2m + 1
-                    // colour of x = 2m (row parity k / KC): a constant after unrolling
-                    const bool c0 = ((k / KC + ZP) & 1) != 0;
-                    v0 = v0 + (c0 ? pr : pl);
-                    v1 = v1 + (c0 ? pl : pr);
+                    // half-sweep 0 overwrites colour CF before anything reads it: only the
+                    // other colour is filled, and CF's zeros where no half-sweep comes
+                    constexpr int C = 1 - CF;
+                    // side of the colour-C cell, x = 2m + sd (row parity k / KC): a constant
+                    // after unrolling
+                    const int sd = (k / KC + ZP + C) & 1;
+                    const float v = xpf[C][k] + (wz0 * q0[sd][k] + wz1 * q1[sd][k]);
+                    base[C * PLANE + e_[k]] = ok ? v : 0.0f;
+                    if (!ok) base[CF * PLANE + e_[k]] = 0.0f;
+                } else {
+                    base[e_[k]] = ok ? xpf[0][k] : 0.0f;
+                    base[PLANE + e_[k]] = ok ? xpf[1][k] : 0.0f;
                 }
-                base[e_[k]] = ok ? v0 : 0.0f;
-                base[PLANE + e_[k]] = ok ? v1 : 0.0f;
             }
         }
     }
@@ -596,7 +599,7 @@ struct Tb2Thread {
     float bv[2][KP];
     double acc[2];
     TbPro<NS, TXP, TY, NTHREADS, PL> pro;  // PRO: the coarse level
-    float xk[2][KP];                       // PRO: x until fill_pro
+    float xk[KP];                          // PRO: x of the colour that half-sweep 0 reads, until fill_pro
 
     __host__ __device__ __forceinline__ void init(float* lds_, const Dims& D_, int bx, int by, const float* xin,
                                                   const float* r, float s_, const float* rinv, int tid_,
@@ -641,8 +644,8 @@ struct Tb2Thread {
         for (int k = 0; k < KP; ++k) {
             xv[0][k] = xv[1][k] = 0.0f;
             if (!ZERO_X) {
-                xv[0][k] = xin[goff[k]];
-                xv[1][k] = xin[n2 + goff[k]];
+                if constexpr (!(PRO && CF == 0)) xv[0][k] = xin[goff[k]];
+                if constexpr (!(PRO && CF == 1)) xv[1][k] = xin[n2 + goff[k]];
             }
             b0[0][k] = r[goff[k]];
             b0[1][k] = r[n2 + goff[k]];
@@ -652,8 +655,7 @@ struct Tb2Thread {
         for (int k = 0; k < KP; ++k) {
             const bool ok = ind[k];
             if constexpr (PRO) {
-                xk[0][k] = xv[0][k];
-                xk[1][k] = xv[1][k];
+                xk[k] = xv[1 - CF][k];
             } else if ((k % KC) * NT + tid < CPOS) {
                 lds[e_[k]] = ok ? xv[0][k] : 0.0f;
                 lds[PLANE + e_[k]] = ok ? xv[1][k] : 0.0f;
@@ -671,12 +673,11 @@ struct Tb2Thread {
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             if ((k % KC) * NT + tid < CPOS) {
-                const bool ok = ind[k];
-                const bool c0 = (k / KC) != 0;
-                const float v0 = xk[0][k] + (c0 ? qv[1][k] : qv[0][k]);
-                const float v1 = xk[1][k] + (c0 ? qv[0][k] : qv[1][k]);
-                lds[e_[k]] = ok ? v0 : 0.0f;
-                lds[PLANE + e_[k]] = ok ? v1 : 0.0f;
+                // half-sweep 0 overwrites colour CF before anything reads it
+                constexpr int C = 1 - CF;
+                const float v = xk[k] + qv[(k / KC + C) & 1][k];
+                lds[C * PLANE + e_[k]] = ind[k] ? v : 0.0f;
+                lds[CF * PLANE + e_[k]] = 0.0f;
             }
         }
     }
