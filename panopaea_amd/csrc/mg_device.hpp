@@ -208,8 +208,9 @@ __device__ __forceinline__ double smooth_half_run(const Dims& D, T* zv, const T*
     return acc;
 }
 
-// q = A p for the x-pair run, with sum(p*q) over its cells in the order
-// (plane, x0 then x1). Each distinct value is loaded once: the pair's x0 and
+// A p for the x-pair run (apply_values: into registers, with p's own values;
+// planes past the last hold values not to be used), and q = A p with sum(p*q)
+// over its cells in the order (plane, x0 then x1). Each distinct value is loaded once: the pair's x0 and
 // x1 on planes z0-1 .. z0+NZ (the run's cells and their z neighbours), and per
 // run plane the x1 of pair m-1, the x0 of pair m+1 and both cells of rows y-1
 // and y+1 (the y neighbours of x0 / x1 are the x0 / x1 of those rows, as the
@@ -221,7 +222,8 @@ __device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0
 __host__ inline void sched_fence() {}
 
 template <typename T, int DIM, int NZ>
-__host__ __device__ __forceinline__ double apply_run(const Dims& D, T* q, const T* p, T dt, int m, int y, int z0) {
+__host__ __device__ __forceinline__ void apply_values(const Dims& D, const T* p, T dt, int m, int y, int z0,
+                                                      T (&q)[NZ][2], T (*pv)[2] = nullptr) {
     const int wh = D.w >> 1, hw = D.h * wh, n2 = D.d * hw;
     const int ml = m > 0 ? m - 1 : m, mr = m + 1 < wh ? m + 1 : m;
     const int yl = y > 0 ? y - 1 : y, yr = y + 1 < D.h ? y + 1 : y;
@@ -272,21 +274,50 @@ __host__ __device__ __forceinline__ double apply_run(const Dims& D, T* q, const 
             yrv[k][c] = ldx(p, iyr[k][c]);
         }
     }
+    // away from the y and z sides (a whole wave on the 64-wide tiles) only x selects
+    const bool inner = y > 0 && y < D.h - 1 && (DIM == 2 || (z0 > 0 && z0 + NZ < D.d));
+    if (inner) {
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            q[k][0] = poisson_inner<T, DIM>(cv[k + 1][0], xl[k], cv[k + 1][1], ylv[k][0], yrv[k][0], cv[k][0],
+                                            cv[k + 2][0], 2 | (m > 0), D.bc, dt);
+            q[k][1] = poisson_inner<T, DIM>(cv[k + 1][1], cv[k + 1][0], xr[k], ylv[k][1], yrv[k][1], cv[k][1],
+                                            cv[k + 2][1], 1 | ((m < wh - 1) << 1), D.bc, dt);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            const RBRow R = rb_row<DIM>(D, z0 + k, y, m);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const T a = c == 0 ? xl[k] : cv[k + 1][0];  // x-1
+                const T b = c == 0 ? cv[k + 1][1] : xr[k];  // x+1
+                q[k][c] = poisson_from<T, DIM>(cv[k + 1][c], a, b, ylv[k][c], yrv[k][c], cv[k][c], cv[k + 2][c],
+                                               c == 0 ? R.has0 : R.has1, D.bc, dt);
+            }
+        }
+    }
+    if (pv)
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            pv[k][0] = cv[k + 1][0];
+            pv[k][1] = cv[k + 1][1];
+        }
+}
+
+template <typename T, int DIM, int NZ>
+__host__ __device__ __forceinline__ double apply_run(const Dims& D, T* q, const T* p, T dt, int m, int y, int z0) {
+    T v[NZ][2], pc[NZ][2];
+    apply_values<T, DIM, NZ>(D, p, dt, m, y, z0, v, pc);
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < NZ; ++k) {
-        const int z = z0 + k;
-        if (z >= D.d) continue;
-        const RBRow R = rb_row<DIM>(D, z, y, m);
+        if (z0 + k >= D.d) continue;
+        const RBRow R = rb_row<DIM>(D, z0 + k, y, m);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const T pc = cv[k + 1][c];
-            const T a = c == 0 ? xl[k] : cv[k + 1][0];  // x-1
-            const T b = c == 0 ? cv[k + 1][1] : xr[k];  // x+1
-            const T v = poisson_from<T, DIM>(pc, a, b, ylv[k][c], yrv[k][c], cv[k][c], cv[k + 2][c],
-                                             c == 0 ? R.has0 : R.has1, D.bc, dt);
-            stx(q, c == 0 ? R.i0 : R.i1, v);
-            s += (double)pc * (double)v;
+            stx(q, c == 0 ? R.i0 : R.i1, v[k][c]);
+            s += (double)pc[k][c] * (double)v[k][c];
         }
     }
     return s;
@@ -343,6 +374,7 @@ __host__ __device__ __forceinline__ double apply_run_y(const Dims& D, T* q, cons
         xr[k] = ldx(p, ir[k]);
     }
     double s = 0.0;
+    const bool inner = y0 > 0 && y0 + NY < D.h;
 #pragma unroll
     for (int k = 0; k < NY; ++k) {
         const int y = y0 + k;
@@ -353,8 +385,9 @@ __host__ __device__ __forceinline__ double apply_run_y(const Dims& D, T* q, cons
             const T pc = cv[k + 1][c];
             const T a = c == 0 ? xl[k] : cv[k + 1][0];  // x-1
             const T b = c == 0 ? cv[k + 1][1] : xr[k];  // x+1
-            const T v = poisson_from<T, 2>(pc, a, b, cv[k][c], cv[k + 2][c], (T)0, (T)0, c == 0 ? R.has0 : R.has1,
-                                           D.bc, dt);
+            const int has = c == 0 ? R.has0 : R.has1;
+            const T v = inner ? poisson_inner<T, 2>(pc, a, b, cv[k][c], cv[k + 2][c], (T)0, (T)0, has, D.bc, dt)
+                              : poisson_from<T, 2>(pc, a, b, cv[k][c], cv[k + 2][c], (T)0, (T)0, has, D.bc, dt);
             stx(q, c == 0 ? R.i0 : R.i1, v);
             s += (double)pc * (double)v;
         }

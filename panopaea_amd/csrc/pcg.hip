@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_apply_dot_rb(Dims D, Grid3 G, T* q, con
                                                       const SolverState* st) {
     if (st->done) return;
     int m, y, zb, L;
-    tile_xyz(G, m, y, zb, L);
+    tile_xyz_stream(G, (int64_t)D.w * D.h * D.d * sizeof(T), m, y, zb, L);
     double s = 0.0;
     if constexpr (DIM == 2) {  // runs of NZ rows (grid3_ap)
         if (m < (D.w >> 1) && y * NZ < D.h) s = apply_run_y<T, NZ>(D, q, p, dt, m, y * NZ);
@@ -692,28 +692,37 @@ static pano_status precond_apply(Ctx* c, const Dims& D, const pano_pcg_params* P
 // ---- mixed precision: FP64 iterative refinement around the FP32 MG-PCG ------------------
 
 // r32 = (float)(b - A x) with the operator and the difference in FP64
-// (red-black layout); partial max |b - A x| in FP64.
-template <int DIM>
+// (red-black layout); partial max |b - A x| in FP64. Runs of NZ planes, every
+// load of a run first (apply_run's values): a loop over the planes waited for
+// each plane's 15 loads before the next one's. 512^3: 751 -> 600 us with the
+// stream order of the tiles; x and b read and r32 written once are 2.7 GB,
+// 435 us at the rate of the streaming kernels (6.2 TB/s). What is left is
+// latency: the run's values take 152 VGPRs, three waves per SIMD.
+template <int DIM, int NZ>
 __global__ __launch_bounds__(256) void k_resid64_rb(Dims D, Grid3 G, float* r32, const double* x, const double* b,
                                                     double dt, double* pmax) {
     int m, y, zb, L;
-    tile_xyz(G, m, y, zb, L);
+    tile_xyz_stream(G, (int64_t)D.w * D.h * D.d * sizeof(double), m, y, zb, L);
     double mx = 0.0;
     if (m < (D.w >> 1) && y < D.h) {
-        const int nz = run_len(D);
-        for (int kz = 0; kz < nz; ++kz) {
-            int z = zb * nz + kz;
-            if (z >= D.d) break;
-            RBRow R = rb_row<DIM>(D, z, y, m);
+        double bv[NZ][2], ax[NZ][2];
+        int i[NZ][2];
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                int i = k == 0 ? R.i0 : R.i1;
-                int has = k == 0 ? R.has0 : R.has1;
-                double n[6];
-                rb_nbrs<double, DIM>(x, R, k, n);
-                double ax = poisson_from<double, DIM>(x[i], n[0], n[1], n[2], n[3], n[4], n[5], has, D.bc, dt);
-                double r = b[i] - ax;
-                r32[i] = (float)r;
+        for (int k = 0; k < NZ; ++k) {
+            const RBRow R = rb_row<DIM>(D, zclamp(D, zb * NZ + k), y, m);
+            i[k][0] = R.i0;
+            i[k][1] = R.i1;
+            bv[k][0] = b[R.i0];
+            bv[k][1] = b[R.i1];
+        }
+        apply_values<double, DIM, NZ>(D, x, dt, m, y, zb * NZ, ax);
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            if (zb * NZ + k >= D.d) continue;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const double r = bv[k][c] - ax[k][c];
+                r32[i[k][c]] = (float)r;
                 mx = absmax_acc(mx, r);
             }
         }
@@ -793,12 +802,14 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
     int outer = 0, inner_total = 0;
     for (;;) {
         // r = b - A x in FP64 (to the FP32 buffer of the inner solve); stop test in FP64
-        if (D.d > 1)
-            hipLaunchKernelGGL(k_resid64_rb<3>, dim3(Gr.nb), dim3(kTX, kTY), 0, s, D, Gr, S.r, (const double*)xx,
+        auto resid = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(Gr.nb), dim3(kTX, kTY), 0, s, D, Gr, S.r, (const double*)xx,
                                (const double*)bb, M->inner.dt, part);
-        else
-            hipLaunchKernelGGL(k_resid64_rb<2>, dim3(Gr.nb), dim3(kTX, kTY), 0, s, D, Gr, S.r, (const double*)xx,
-                               (const double*)bb, M->inner.dt, part);
+        };
+        if (D.d <= 1) resid(k_resid64_rb<2, 1>);
+        else if (run_len(D) == 4) resid(k_resid64_rb<3, 4>);
+        else if (run_len(D) == 2) resid(k_resid64_rb<3, 2>);
+        else resid(k_resid64_rb<3, 1>);
         launch_finalize(s, FIN_RNORM, part, nullptr, Gr.nb, st2, cfg2, 1);
         PANO_HIP(hipMemcpyAsync(&hs[1], st2, sizeof(SolverState), hipMemcpyDeviceToHost, s));
         PANO_HIP(hipStreamSynchronize(s));
