@@ -252,7 +252,20 @@ static void smooth_tb(Ctx* c, const char* name, double bytes, const Dims& D, con
 // restriction. It streams plane by plane, so a workgroup's time is a chain of
 // load latencies: on levels below 2^23 cells the two separate kernels (more
 // workgroups, no chain) are faster.
-constexpr int kRrTX = 32, kRrTY = 8, kRrWant = 1024, kRrKmin = 2, kRrPD = 1;
+constexpr int kRrWant = 512, kRrKmin = 2, kRrPD = 1;
+// Its tiles, coarse cells in x by rows, 512 threads and two workgroups per CU
+// each. A tile's rows are read with two pairs more on each side, which are two
+// more 128-byte lines per colour, so its L2 misses fall with its width: at 512^3
+// 32 x 8 tiles fetched 2.1 times the field and ran at the memory's rate.
+// Level 0 of 512^3 / 256^3, us: 32 x 8 381 / 42, 32 x 16 343 / 36, 64 x 8
+// 304 / 35, 64 x 16 (one workgroup per CU) 304 / 36, 64 x 4 341 / 43; twice
+// the workgroups in shorter chunks 295 / 41. Wide tiles, unless the level's
+// edges leave them more than a tenth more padded cells than narrow ones.
+constexpr int kRrWideX = 64, kRrWideY = 8, kRrNarrowX = 32, kRrNarrowY = 16;
+inline bool rr_wide(const Dims& Dc) {
+    auto padded = [&](int tx, int ty) { return (int64_t)((Dc.w + tx - 1) / tx * tx) * ((Dc.h + ty - 1) / ty * ty); };
+    return 10 * padded(kRrWideX, kRrWideY) <= 11 * padded(kRrNarrowX, kRrNarrowY);
+}
 inline bool rr_on(bool enabled, const Dims& D) {
     return enabled && D.d > 1 && (int64_t)D.d * D.h * D.w >= (int64_t(1) << 23);
 }
@@ -290,9 +303,15 @@ static void resrestrict2(Ctx* c, const char* name, double bytes, const Dims& D, 
 template <int LC>
 static void resrestrict(Ctx* c, const char* name, double bytes, const Dims& D, const Dims& Dc, const float* z,
                         const float* b, float* rc, float s, const SolverState* st) {
-    const RrGrid g = rr_grid<kRrTX, kRrTY>(Dc, kRrWant, kRrKmin);
-    klaunch(c, name, bytes, k_resrestrict<kRrTX, kRrTY, LC>, dim3(g.nb), dim3(kRrTX * kRrTY), D, Dc, g, z, b, rc, s,
-            st);
+    auto launch = [&](auto kern, const RrGrid& g, int nt) {
+        klaunch(c, name, bytes, kern, dim3(g.nb), dim3(nt), D, Dc, g, z, b, rc, s, st);
+    };
+    if (rr_wide(Dc))
+        launch(k_resrestrict<kRrWideX, kRrWideY, LC>, rr_grid<kRrWideX, kRrWideY>(Dc, kRrWant, kRrKmin),
+               kRrWideX * kRrWideY);
+    else
+        launch(k_resrestrict<kRrNarrowX, kRrNarrowY, LC>, rr_grid<kRrNarrowX, kRrNarrowY>(Dc, kRrWant, kRrKmin),
+               kRrNarrowX * kRrNarrowY);
 }
 
 // ---- a level's legs as one launch each (mg_leg.hpp) ------------------------------------

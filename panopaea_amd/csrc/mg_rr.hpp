@@ -107,12 +107,12 @@ struct RrThread {
     bool zin[KZ];
     float zpf[PD][2][KZ];
     bool zok[PD];
-    // residual positions
-    int rzi[KR];   // index in a z colour plane
-    int ridx[KR];  // index in a residual colour plane
-    int roff[KR];
-    int rbits[KR]; // neighbour bits of x0 (bits 0..3) and x1 (bits 8..11), x and y only
-    int ryp[KR];   // row parity
+    // residual positions. Index 0 of an array is the colour of the row's parity
+    // (x0's colour on even planes, x1's on odd ones), 1 the other colour.
+    int rzi[2][KR];     // index in a z plane
+    int ridx[2][KR];    // index in a residual plane
+    int roff[2][KR];    // index in a plane of the field
+    float rnc[2][KR];   // x and y neighbours (sides with a value) of x0 and of x1
     float bpf[PD][2][KR];
     // coarse column
     int I, J, rp, rr0;
@@ -159,13 +159,20 @@ struct RrThread {
             const int e = tid + k * NT;
             int row, pr;
             S::template pos_of<1>(e < RPLANE ? e : 0, RH, row, pr);
-            ridx[k] = e < RPLANE ? row * RW + pr : e;
+            const int ri = e < RPLANE ? row * RW + pr : e;
             const int y = 2 * J0 - 1 + row, m = I0 - 1 + pr;
-            rzi[k] = (row + 1) * ZW + pr + 1;
-            roff[k] = y >= 0 && y < D.h && m >= 0 && m < wh ? y * wh + m : 0;
+            const int zi = (row + 1) * ZW + pr + 1;
+            const int ro = y >= 0 && y < D.h && m >= 0 && m < wh ? y * wh + m : 0;
+            const int c = y & 1;
+            rzi[0][k] = c * ZS + zi;
+            rzi[1][k] = (1 - c) * ZS + zi;
+            ridx[0][k] = c * RS + ri;
+            ridx[1][k] = (1 - c) * RS + ri;
+            roff[0][k] = c * n2 + ro;
+            roff[1][k] = (1 - c) * n2 + ro;
             const int yb = ((y > 0) << 2) | ((y < D.h - 1) << 3);
-            rbits[k] = (yb | (m > 0) | 2) | ((yb | 1 | ((m < wh - 1) << 1)) << 8);
-            ryp[k] = y & 1;
+            rnc[0][k] = (float)ncount_bits<2>(yb | (m > 0) | 2, D.bc);
+            rnc[1][k] = (float)ncount_bits<2>(yb | 1 | ((m < wh - 1) << 1), D.bc);
         }
         const int tx = tid % TXC, tyy = tid / TXC;
         I = I0 + tx;
@@ -179,9 +186,21 @@ struct RrThread {
         own = I < Dc.w && J < Dc.h;
         ty[0] = ty[1] = ty[2] = ty[3] = 0.0f;
     }
-    __host__ __device__ __forceinline__ int slot(int p) const { return (p - pf0 + 1) % S::ZSLOTS; }
-    // the residual plane buffer of step p
-    __host__ __device__ __forceinline__ float* rbuf(int p) const { return rl + ((p - pf0) & 1) * 2 * RS; }
+    // SJ >= 0: the step p - pf0 modulo 4, a constant of the unrolled loop
+    // (rr_steps); with it the slots, the buffers and the plane's parity (pf0 is
+    // odd) are constants too, and LDS addresses of one step differ from
+    // another's by immediate offsets only. SJ < 0: from p.
+    template <int SJ>
+    __host__ __device__ __forceinline__ int step(int p) const {
+        return SJ >= 0 ? SJ : (p - pf0) % S::ZSLOTS;
+    }
+    // z slot of the plane `ahead` planes past that of step j
+    __host__ __device__ __forceinline__ float* zslot(int j, int ahead) const {
+        return zl + ((j + 1 + ahead) % S::ZSLOTS) * 2 * ZS;
+    }
+    // the residual plane buffer of step j
+    __host__ __device__ __forceinline__ float* rbuf(int j) const { return rl + (j & 1) * 2 * RS; }
+    __host__ __device__ static constexpr int parity(int j) { return (j + 1) & 1; }
     __host__ __device__ __forceinline__ const float* plane_ptr(const float* f, int p) const {
         return f + (p < 0 ? 0 : (p >= D.d ? D.d - 1 : p)) * hw;
     }
@@ -199,8 +218,7 @@ struct RrThread {
         }
     }
     template <int Q>
-    __host__ __device__ __forceinline__ void fill_z(int p) {
-        float* base = zl + slot(p) * 2 * ZS;
+    __host__ __device__ __forceinline__ void fill_z(float* base) {
 #pragma unroll
         for (int k = 0; k < KZ; ++k) {
             const bool ok = zok[Q] && zin[k];
@@ -211,11 +229,10 @@ struct RrThread {
     template <int Q>
     __host__ __device__ __forceinline__ void load_b(int p) {
         const float* p0 = plane_ptr(b, p);
-        const float* p1 = p0 + n2;
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            bpf[Q][0][k] = ldx(p0, roff[k]);
-            bpf[Q][1][k] = ldx(p1, roff[k]);
+            bpf[Q][0][k] = ldx(p0, roff[0][k]);
+            bpf[Q][1][k] = ldx(p0, roff[1][k]);
         }
     }
     // b of plane pf0+Q and z of plane pf0+3+Q into set Q, for Q < PD: the
@@ -253,53 +270,49 @@ struct RrThread {
                 zpf[0][0][k] = v[j][0][k];
                 zpf[0][1][k] = v[j][1][k];
             }
-            fill_z<0>(pf0 - 1 + j);
+            fill_z<0>(zslot(0, j - 1));
         }
         load_ahead<0>();
     }
-    // residual of fine plane p into the residual plane rdst (both colours),
-    // from the z planes zc (p), zm (p-1), zp (p+1) in LDS and b of plane p
+    // residual of fine plane p (parity cz) into the residual plane rdst (both
+    // colours), from the z planes zc (p), zm (p-1), zp (p+1) in LDS and b of
+    // plane p. The neighbour count is a sum of small whole numbers, exact in f32.
     __host__ __device__ __forceinline__ void residual_plane(float* rdst, const float* zc, const float* zm,
-                                                            const float* zp, int p, const float (&bb)[2][KR]) const {
-        const int zb = ((p > 0) << 4) | ((p < D.d - 1) << 5);
-        const int cz = p & 1;
+                                                            const float* zp, int p, int cz,
+                                                            const float (&bb)[2][KR]) const {
+        const float ncz = (float)__builtin_popcount(
+            (unsigned)(((((p > 0) << 4) | ((p < D.d - 1) << 5)) | D.bc) & 0x30));
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int c0 = cz ^ ryp[k];  // colour of the pair's even cell x0
-            const int c1 = 1 - c0;
-            const int e = rzi[k];
-            const float* o0 = zc + c1 * ZS;  // x0's neighbours in the plane, and x1
-            const float* o1 = zc + c0 * ZS;  // x1's neighbours in the plane, and x0
+            const int e1 = rzi[cz][k];      // x0, and x1's neighbours in the plane
+            const int e0 = rzi[1 - cz][k];  // x1, and x0's neighbours in the plane
             float n0[6], n1[6];
-            n0[0] = o0[e - 1];
-            n0[1] = o0[e];
-            n0[2] = o0[e - ZW];
-            n0[3] = o0[e + ZW];
-            n0[4] = zm[c1 * ZS + e];
-            n0[5] = zp[c1 * ZS + e];
-            n1[0] = o1[e];
-            n1[1] = o1[e + 1];
-            n1[2] = o1[e - ZW];
-            n1[3] = o1[e + ZW];
-            n1[4] = zm[c0 * ZS + e];
-            n1[5] = zp[c0 * ZS + e];
-            const float z0 = o1[e], z1 = o0[e];
-            const float b0 = c0 ? bb[1][k] : bb[0][k], b1 = c0 ? bb[0][k] : bb[1][k];
-            const int h0 = (rbits[k] & 0xF) | zb, h1 = ((rbits[k] >> 8) & 0xF) | zb;
-            const float a0 = s * ((float)ncount_bits<3>(h0, D.bc) * z0 - nsum<float, 3>(n0));
-            const float a1 = s * ((float)ncount_bits<3>(h1, D.bc) * z1 - nsum<float, 3>(n1));
-            rdst[c0 * RS + ridx[k]] = b0 - a0;
-            rdst[c1 * RS + ridx[k]] = b1 - a1;
+            n0[0] = zc[e0 - 1];
+            n0[1] = zc[e0];
+            n0[2] = zc[e0 - ZW];
+            n0[3] = zc[e0 + ZW];
+            n0[4] = zm[e0];
+            n0[5] = zp[e0];
+            n1[0] = zc[e1];
+            n1[1] = zc[e1 + 1];
+            n1[2] = zc[e1 - ZW];
+            n1[3] = zc[e1 + ZW];
+            n1[4] = zm[e1];
+            n1[5] = zp[e1];
+            const float a0 = s * ((rnc[0][k] + ncz) * zc[e1] - nsum<float, 3>(n0));
+            const float a1 = s * ((rnc[1][k] + ncz) * zc[e0] - nsum<float, 3>(n1));
+            rdst[ridx[cz][k]] = bb[cz][k] - a0;
+            rdst[ridx[1 - cz][k]] = bb[1 - cz][k] - a1;
         }
     }
-    // fine plane p of the residual plane rsrc restricted along x, then y, for
-    // the thread's coarse column
-    __host__ __device__ __forceinline__ float restrict_xy(const float* rsrc, int p) const {
+    // the residual plane rsrc (of a fine plane of parity cz) restricted along x,
+    // then y, for the thread's coarse column
+    __host__ __device__ __forceinline__ float restrict_xy(const float* rsrc, int cz) const {
         float t[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int row = rr0 + q;                 // fine row 2J-1+q
-            const int ce = (2 * J - 1 + q + p) & 1;  // colour of the fine x = 2I
+            const int row = rr0 + q;         // fine row 2J-1+q
+            const int ce = (q + 1 + cz) & 1;  // colour of the fine x = 2I
             const float* pe = rsrc + ce * RS + row * RW + rp;
             const float* po = rsrc + (1 - ce) * RS + row * RW + rp;
             t[q] = r1(po[-1], pe[0], po[0], pe[1], hmI, hpI);
@@ -308,27 +321,31 @@ struct RrThread {
     }
     // residual of plane p (b in register set Q) into LDS (nothing for planes
     // outside the grid); then b of plane p+PD into set Q
-    template <int Q>
+    template <int Q, int SJ = -1>
     __host__ __device__ __forceinline__ void phase1(int p) {
+        const int j = step<SJ>(p);
         if (p >= 0 && p < D.d)
-            residual_plane(rbuf(p), zl + slot(p) * 2 * ZS, zl + slot(p - 1) * 2 * ZS, zl + slot(p + 1) * 2 * ZS,
-                           p, bpf[Q]);
+            residual_plane(rbuf(j), zslot(j, 0), zslot(j, -1), zslot(j, 1), p, parity(j), bpf[Q]);
         load_b<Q>(p + PD);
     }
     // plane p restricted along x and y into the ring; r_c(K) once plane
     // 2K+2 is in; then the slot of plane p+3 (that of plane p-1, last read by
     // phase 1 of this step) from set Q and z of plane p+3+PD into set Q
-    template <int Q>
+    template <int Q, int SJ = -1>
     __host__ __device__ __forceinline__ void phase2(int p) {
+        const int j = step<SJ>(p);
         ty[0] = ty[1];
         ty[1] = ty[2];
         ty[2] = ty[3];
-        ty[3] = p >= 0 && p < D.d ? restrict_xy(rbuf(p), p) : 0.0f;
-        // r_c(K) for p = 2K+2 (an always-issued store, dropped on other steps)
-        const bool st = p >= 2 * K0 + 2 && !(p & 1);
-        const int K = st ? p / 2 - 1 : K0;
-        st_if(rco, own ? cidx<LC>(Dc, K, J, I) : 0, r1(ty[0], ty[1], ty[2], ty[3], K > 0, K < Dc.d - 1), st && own);
-        fill_z<Q>(p + 3);
+        ty[3] = p >= 0 && p < D.d ? restrict_xy(rbuf(j), parity(j)) : 0.0f;
+        // r_c(K) for p = 2K+2 (an always-issued store, dropped on the first such step)
+        if (parity(j) == 0) {
+            const bool st = p >= 2 * K0 + 2;
+            const int K = st ? p / 2 - 1 : K0;
+            st_if(rco, own ? cidx<LC>(Dc, K, J, I) : 0, r1(ty[0], ty[1], ty[2], ty[3], K > 0, K < Dc.d - 1),
+                  st && own);
+        }
+        fill_z<Q>(zslot(j, 3));
         load_z<Q>(p + 3 + PD);
     }
 };
@@ -367,27 +384,21 @@ struct Rr2Thread : RrThread<TXC, TYC, LC, 1> {
         const float* zc = B::zl;
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int c0 = B::ryp[k];  // colour of the pair's even cell x0 (plane 0)
-            const int c1 = 1 - c0;
-            const int e = B::rzi[k];
-            const float* o0 = zc + c1 * ZS;
-            const float* o1 = zc + c0 * ZS;
+            const int e1 = B::rzi[0][k];  // x0, and x1's neighbours
+            const int e0 = B::rzi[1][k];  // x1, and x0's neighbours
             float n0[4], n1[4];
-            n0[0] = o0[e - 1];
-            n0[1] = o0[e];
-            n0[2] = o0[e - ZW];
-            n0[3] = o0[e + ZW];
-            n1[0] = o1[e];
-            n1[1] = o1[e + 1];
-            n1[2] = o1[e - ZW];
-            n1[3] = o1[e + ZW];
-            const float z0 = o1[e], z1 = o0[e];
-            const float b0 = c0 ? B::bpf[0][1][k] : B::bpf[0][0][k], b1 = c0 ? B::bpf[0][0][k] : B::bpf[0][1][k];
-            const int h0 = B::rbits[k] & 0xF, h1 = (B::rbits[k] >> 8) & 0xF;
-            const float a0 = B::s * ((float)ncount_bits<2>(h0, B::D.bc) * z0 - nsum<float, 2>(n0));
-            const float a1 = B::s * ((float)ncount_bits<2>(h1, B::D.bc) * z1 - nsum<float, 2>(n1));
-            B::rl[c0 * RS + B::ridx[k]] = b0 - a0;
-            B::rl[c1 * RS + B::ridx[k]] = b1 - a1;
+            n0[0] = zc[e0 - 1];
+            n0[1] = zc[e0];
+            n0[2] = zc[e0 - ZW];
+            n0[3] = zc[e0 + ZW];
+            n1[0] = zc[e1];
+            n1[1] = zc[e1 + 1];
+            n1[2] = zc[e1 - ZW];
+            n1[3] = zc[e1 + ZW];
+            const float a0 = B::s * (B::rnc[0][k] * zc[e1] - nsum<float, 2>(n0));
+            const float a1 = B::s * (B::rnc[1][k] * zc[e0] - nsum<float, 2>(n1));
+            B::rl[B::ridx[0][k]] = B::bpf[0][0][k] - a0;
+            B::rl[B::ridx[1][k]] = B::bpf[0][1][k] - a1;
         }
     }
     __host__ __device__ __forceinline__ void restrict_store() {
@@ -418,10 +429,11 @@ __device__ __forceinline__ void rr2_workgroup(float* lds, const Dims& D, const D
 // barrier behind), and writes the other residual buffer, last read by phase
 // 2 of step p-1; phase 2 of step p fills the slot of plane p-1, last read by
 // phase 1 of step p. So one barrier per step.
-template <int PD, typename TH, int... Q>
-__device__ __forceinline__ void rr_steps(TH& th, int& p, int p1, std::integer_sequence<int, Q...>) {
-    ((p <= p1 ? (__syncthreads(), th.template phase2<Q>(p),
-                 (p + 1 <= p1 ? th.template phase1<(Q + 1) % PD>(p + 1) : (void)0), ++p)
+// The steps j = 0 .. 3 of a round are unrolled (TH::step).
+template <int PD, typename TH, int... J>
+__device__ __forceinline__ void rr_steps(TH& th, int& p, int p1, std::integer_sequence<int, J...>) {
+    ((p <= p1 ? (__syncthreads(), th.template phase2<J % PD, J>(p),
+                 (p + 1 <= p1 ? th.template phase1<(J + 1) % PD, (J + 1) % 4>(p + 1) : (void)0), ++p)
               : p),
      ...);
 }
@@ -435,8 +447,9 @@ __device__ __forceinline__ void rr_workgroup(float* lds, const Dims& D, const Di
     th.prologue();
     __syncthreads();
     int p = th.pf0;
-    th.template phase1<0>(p);
-    while (p <= th.pf1) rr_steps<PD>(th, p, th.pf1, std::make_integer_sequence<int, PD>{});
+    th.template phase1<0, 0>(p);
+    static_assert(4 % PD == 0, "a round of steps ends on register set 0");
+    while (p <= th.pf1) rr_steps<PD>(th, p, th.pf1, std::make_integer_sequence<int, 4>{});
 }
 
 }  // namespace pano
