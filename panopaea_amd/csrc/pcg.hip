@@ -160,6 +160,7 @@ struct Solver {
     // `auxiliary` holds both (pcg.rs:51,65)
     T *x, *r, *aux, *p, *q;
     int it;  // iterations enqueued in this solve
+    bool x_final = true; // the loop applies the last update's x step (false: the caller's next pass over x does)
     ClPlan cl;           // the one-kernel loop (cl.wgs == 0: the launches)
     ClSlots* slots;
     unsigned spin;
@@ -420,8 +421,9 @@ static pano_status solver_loop(Solver<T>* S, int max_iterations, int every, cons
         return PANO_OK;
     };
     auto epilogue = [&]() -> pano_status {
-        hipLaunchKernelGGL((k_x_final<T>), dim3(S->nflat), dim3(kBlock), 0, c->stream, S->n, S->x,
-                           (const T*)S->p, (const SolverState*)S->st);
+        if (S->x_final)
+            hipLaunchKernelGGL((k_x_final<T>), dim3(S->nflat), dim3(kBlock), 0, c->stream, S->n, S->x,
+                               (const T*)S->p, (const SolverState*)S->st);
         PANO_HIP(hipGetLastError());
         return epi();
     };
@@ -731,21 +733,69 @@ __global__ __launch_bounds__(256) void k_resid64_rb(Dims D, Grid3 G, float* r32,
     if (threadIdx.x == 0 && threadIdx.y == 0) pmax[L] = t;
 }
 
-// x += (double)e
-__global__ __launch_bounds__(256) void k_add_correction(int64_t n, double* x, const float* e) {
-    int64_t base = (int64_t)blockIdx.x * kFlatPer + threadIdx.x;
+// Sums of b, one partial per workgroup (the mean's input).
+__global__ __launch_bounds__(256) void k_sum64(int64_t n, const double* b, double* psum) {
+    double t, m;
+    flat_stats(blockIdx.x, n, b, &t, &m);
+    if (threadIdx.x == 0) psum[blockIdx.x] = t;
+}
+
+// The start of the refinement from x = 0: b - mean (mean null: b as it is) and,
+// as b - A 0 is b, the first residual r32 = (float)b with max|b| in the same
+// pass. 512^3: the zeroing of x, the removal of the mean and the first
+// residual were three passes of 364 + 367 + 600 us.
+__global__ __launch_bounds__(256) void k_start64(int64_t n, double* b, float* r32, const SolverState* mean,
+                                                 double* pmax) {
+    const int64_t base = (int64_t)blockIdx.x * kFlatPer + threadIdx.x;
+    const double mu = mean ? mean->mean : 0.0;
+    double v[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {  // all loads before any store (clamped, valid indices)
+        const int64_t i = base + (int64_t)k * kBlock;
+        v[k] = b[i < n ? i : n - 1];
+    }
+    double m = 0.0;
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int64_t i = base + (int64_t)k * kBlock;
+        if (i < n) {
+            if (mean) {
+                v[k] = v[k] - mu;
+                b[i] = v[k];
+            }
+            r32[i] = (float)v[k];
+            m = absmax_acc(m, v[k]);
+        }
+    }
+    const double t = block_max(m);
+    if (threadIdx.x == 0) pmax[blockIdx.x] = t;
+}
+
+// x += e in FP64, e the inner solve's solution with its last update's step
+// still to add (k_x_final's expression, in FP32). FIRST: x was 0 and is not
+// read (nor was it written). Streams at the copy rate of these kernels: 512^3
+// e, p and x read and x written once are 3.2 GB. Two passes (the step, then
+// the sum) took 315 + 500 us.
+template <bool FIRST>
+__global__ __launch_bounds__(256) void k_add_correction(int64_t n, double* x, const float* e, const float* p,
+                                                        const SolverState* st) {
+    const int64_t base = (int64_t)blockIdx.x * kFlatPer + threadIdx.x;
+    const bool step = st->xit < st->iter;
+    const double alpha = st->alpha;
     double xv[kItems];
-    float ev[kItems];
+    float ev[kItems], pv[kItems];
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {  // all loads before any store (clamped, valid indices)
         const int64_t i = base + (int64_t)k * kBlock, j = i < n ? i : n - 1;
-        xv[k] = x[j];
+        xv[k] = FIRST ? 0.0 : x[j];
         ev[k] = e[j];
+        pv[k] = step ? p[j] : 0.0f;
     }
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
         const int64_t i = base + (int64_t)k * kBlock;
-        if (i < n) x[i] = xv[k] + (double)ev[k];
+        const float el = step ? (float)((double)ev[k] + alpha * (double)pv[k]) : ev[k];
+        if (i < n) x[i] = xv[k] + (double)el;
     }
 }
 
@@ -775,6 +825,7 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
     S.p = (float*)pp;
     S.q = nullptr;
     S.x = (float*)e;
+    S.x_final = false;
     SolverState* st2 = (SolverState*)st2v;
     double* part = (double*)part2;
     double* bb = (double*)b64;
@@ -789,28 +840,28 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
     cfg2.round_f32 = 0;
     Grid3 Gn = grid3(D.w, D.h, D.d);
     hipLaunchKernelGGL((k_to_rb<double>), dim3(Gn.nb), dim3(kTX, kTY), 0, s, D, Gn, bb, b);
-    hipLaunchKernelGGL((k_zero_stats<double>), dim3(S.nflat), dim3(kBlock), 0, s, n, xx, (const double*)bb, S.part0,
-                       part);
     if (cfg2.remove_mean) {
+        hipLaunchKernelGGL(k_sum64, dim3(S.nflat), dim3(kBlock), 0, s, n, (const double*)bb, S.part0);
         launch_finalize(s, FIN_STATS, S.part0, nullptr, S.nflat, st2, cfg2, 0);
-        hipLaunchKernelGGL((k_sub_mean<double>), dim3(S.nflat), dim3(kBlock), 0, s, n, bb, (const SolverState*)st2,
-                           part);
     }
+    hipLaunchKernelGGL(k_start64, dim3(S.nflat), dim3(kBlock), 0, s, n, bb, S.r,
+                       (const SolverState*)(cfg2.remove_mean ? st2 : nullptr), part);
     launch_finalize(s, FIN_THRESH, part, nullptr, S.nflat, st2, cfg2, 1);
     SolverState* hs = c->host_state;
     const std::string key = hint_key(D, &ip, sizeof(float));
     int outer = 0, inner_total = 0;
     for (;;) {
-        // r = b - A x in FP64 (to the FP32 buffer of the inner solve); stop test in FP64
+        // r = b - A x in FP64 (to the FP32 buffer of the inner solve; x = 0: k_start64's); stop test in FP64
         auto resid = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(Gr.nb), dim3(kTX, kTY), 0, s, D, Gr, S.r, (const double*)xx,
                                (const double*)bb, M->inner.dt, part);
         };
-        if (D.d <= 1) resid(k_resid64_rb<2, 1>);
+        if (outer == 0) {
+        } else if (D.d <= 1) resid(k_resid64_rb<2, 1>);
         else if (run_len(D) == 4) resid(k_resid64_rb<3, 4>);
         else if (run_len(D) == 2) resid(k_resid64_rb<3, 2>);
         else resid(k_resid64_rb<3, 1>);
-        launch_finalize(s, FIN_RNORM, part, nullptr, Gr.nb, st2, cfg2, 1);
+        launch_finalize(s, FIN_RNORM, part, nullptr, outer == 0 ? S.nflat : Gr.nb, st2, cfg2, 1);
         PANO_HIP(hipMemcpyAsync(&hs[1], st2, sizeof(SolverState), hipMemcpyDeviceToHost, s));
         PANO_HIP(hipStreamSynchronize(s));
         if (hs[1].done) break;
@@ -819,9 +870,15 @@ static pano_status mixed_solve(Ctx* c, const Dims& D, const pano_mixed_params* M
         PANO_CHECK(solver_loop<float>(&S, ip.max_iterations, ip.check_every, &key, []() { return PANO_OK; }));
         if (hs[0].nonfinite) return fail(PANO_ERR_NONFINITE, "non-finite value in the inner solve");
         inner_total += hs[0].iter;
+        auto add = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(S.nflat), dim3(kBlock), 0, s, n, xx, (const float*)S.x, (const float*)S.p,
+                               (const SolverState*)S.st);
+        };
+        if (outer == 0) add(k_add_correction<true>);
+        else add(k_add_correction<false>);
         ++outer;
-        hipLaunchKernelGGL(k_add_correction, dim3(S.nflat), dim3(kBlock), 0, s, n, xx, (const float*)S.x);
     }
+    if (outer == 0) PANO_HIP(hipMemsetAsync(xx, 0, n * sizeof(double), s));  // nothing to correct: x = 0
     hipLaunchKernelGGL((k_from_rb<double>), dim3(Gn.nb), dim3(kTX, kTY), 0, s, D, Gn, x, (const double*)xx);
     PANO_HIP(hipStreamSynchronize(s));
     PANO_HIP(hipGetLastError());
