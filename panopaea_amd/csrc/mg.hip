@@ -383,42 +383,6 @@ static bool leg_up_on(const MG<T>* m, int l) {
 }
 
 // ---- coarsest level: fast diagonalisation in FP64 (natural layout) ---------------------
-// out[line j] = sum_k V[j*n+k] * in[line k] (inverse=1) or
-// out[line k] = sum_j V[j*n+k] * in[line j] (inverse=0), along `axis`.
-// With scale_mode, the forward result is divided by s*(lx+ly+lz) (0 for a
-// null mode).
-template <typename Tin, typename Tout>
-__global__ __launch_bounds__(256) void k_fdm_axis(int nx, int ny, int nz, int axis, int inverse,
-                                                  const Tin* in, Tout* out, const double* V,
-                                                  int scale_mode, const double* lx, const double* ly,
-                                                  const double* lz, double s, double lam_eps,
-                                                  const SolverState* st) {
-    if (st->done) return;
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t ntot = (int64_t)nx * ny * nz;
-    if (t >= ntot) return;
-    int ix = (int)(t % nx);
-    int64_t r = t / nx;
-    int iy = (int)(r % ny);
-    int iz = (int)(r / ny);
-    int n, pos;
-    int64_t stride, base;
-    if (axis == 0) { n = nx; pos = ix; stride = 1; base = t - ix; }
-    else if (axis == 1) { n = ny; pos = iy; stride = nx; base = t - (int64_t)iy * nx; }
-    else { n = nz; pos = iz; stride = (int64_t)nx * ny; base = t - (int64_t)iz * nx * ny; }
-    double acc = 0.0;
-    if (inverse) {
-        for (int k = 0; k < n; ++k) acc += V[pos * n + k] * (double)in[base + k * stride];
-    } else {
-        for (int j = 0; j < n; ++j) acc += V[j * n + pos] * (double)in[base + j * stride];
-    }
-    if (scale_mode) {
-        double lam = lx[ix] + ly[iy] + (lz ? lz[iz] : 0.0);
-        acc = lam > lam_eps ? acc / (s * lam) : 0.0;
-    }
-    out[t] = (Tout)acc;
-}
-
 // 1D operator along one axis with n cells: diag = (i>0 ? 1 : lo) + (i<n-1 ? 1 : hi),
 // off-diagonal -1 (lo/hi = 1 for an open side). Closed-form eigenpairs:
 //  wall/wall: cos(pi k (j+1/2)/n),            lambda = 2 - 2 cos(pi k/n)
@@ -640,186 +604,202 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_zcol(int nx, int ny, int nz
     fdm_zcol_body(fdm_lds, nx, ny, nz, blockIdx.x, data, Vz, lx, ly, lz, s, eps);
 }
 
-// ---- 3D coarsest level over many workgroups -------------------------------------------
-// The three passes of k_fdm_plane (forward), k_fdm_zcol and k_fdm_plane
-// (inverse), each split over the index that its output sums leave free, so a
-// 32^3 level runs on 256 workgroups of 128 threads instead of 32 of 1024:
-//  forward: plane K, a block of columns i: x for those columns (every row),
-//           then y for them;
-//  z:       row j, a block of columns i: z forward, divide, z inverse;
-//  inverse: plane K, a block of rows j: y for those rows (every column),
-//           then x for them.
-// Every output is the same sum, in the same order (q = 0 .. n-1 from 0), of
-// the same products as in lds_axis, so the results are those of the
-// one-workgroup-per-plane kernels bit for bit. Bases are staged in LDS when
-// they fit in kFdmSplitV doubles (else read from global memory).
-constexpr int kFdmSplitThreads = 128;
-constexpr int kFdmSplitV = 4096;
-// outputs per line block: lines of n outputs per workgroup
-__host__ __device__ inline int fdm_split_w(int n) {
-    const int w = kFdmSplitThreads / n;
-    return w < 1 ? 1 : w;
-}
-// doubles staged for two bases of sizes n0^2 and n1^2 (the first, then the
-// second if both fit), as the kernels below stage them
-__host__ __device__ inline int fdm_split_cap(int n0, int n1) {
-    const int a = n0 * n0 <= kFdmSplitV ? n0 * n0 : 0;
-    const int b = a + n1 * n1 <= kFdmSplitV ? n1 * n1 : 0;
-    return a + b;
-}
-inline size_t fdm_split_lds_fwd(int nx, int ny) {
-    return (size_t)(nx * ny + ny * fdm_split_w(ny) + fdm_split_cap(nx, ny)) * sizeof(double);
-}
-inline size_t fdm_split_lds_z(int nz) {
-    return (size_t)(2 * nz * fdm_split_w(nz) + fdm_split_cap(nz, 0)) * sizeof(double);
-}
-inline size_t fdm_split_lds_inv(int nx, int ny) {
-    return (size_t)(nx * ny + nx * fdm_split_w(nx) + fdm_split_cap(ny, nx)) * sizeof(double);
-}
+// ---- 3D coarsest level: FP64 matrix products on the matrix cores -----------------------
+// The six products of the solve, x, y, z forward, the division, z, y, x inverse,
+// in 16 x 16 tiles of v_mfma_f64_16x16x4 (mfma_tile). Every output is the same
+// chain of fused multiply-adds in the same order (q = 0 .. n-1 from 0) as
+// lds_axis's, so the results are those of k_fdm_plane / k_fdm_zcol bit for bit.
+// With a sum per thread, two LDS reads per product bounded the passes.
+//
+// Three launches for any size, each two products with the first one's result
+// in LDS, split over the index both leave free (64^3: 256 workgroups each):
+//  forward: plane K, 16 columns i: x for them (every row), then y;
+//  z:       16 cells of a plane: z forward, divide, z inverse;
+//  inverse: plane K, 16 rows j: y for them (every column), then x.
+// 64^3 53 + 28 + 49 us with a sum per thread, 7 + 7 + 9 now; 32^3 6.4 + 5.8 +
+// 5.4, now 4.6 + 4.6 + 4.8 (launch and two rounds of loads).
+constexpr int kFdm3Threads = 256;
+constexpr int kFdm3P = 17;  // row length in LDS of a block of 16 columns
+inline size_t fdm3_lds_cols(int n) { return (size_t)((n + 15) / 16 * 16) * kFdm3P * sizeof(double); }
+__host__ __device__ inline int fdm3_row(int nx) { return (nx + 15) / 16 * 16 + 2; }
 
-// forward x then y of plane K, columns [i0, i0 + nc): in -> out (double)
+// forward x then y of plane K, columns [i0, i0 + 16): in -> out (double)
 template <typename Tin>
-__global__ __launch_bounds__(kFdmSplitThreads) void k_fdm_fwd_cols(int nx, int ny, const Tin* in, double* out,
-                                                                   const double* Vx, const double* Vy,
-                                                                   const SolverState* st) {
+__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_fwd(int nx, int ny, const Tin* in, double* out,
+                                                           const double* Vx, const double* Vy,
+                                                           const SolverState* st) {
     if (st->done) return;
     extern __shared__ double fdm_lds[];
-    const int cw = fdm_split_w(ny), ncb = (nx + cw - 1) / cw;
-    const int K = blockIdx.x / ncb, i0 = (blockIdx.x - K * ncb) * cw;
-    const int nc = imin(cw, nx - i0), P = nx * ny;
-    double* a = fdm_lds;   // the plane
-    double* t = a + P;     // its x transform, columns i0.. : t[q * cw + il]
-    double* vs = t + ny * cw;
-    const Tin* src = in + (int64_t)K * P;
-    // the plane and the bases that fit (Vx first, then Vy: fdm_split_cap),
-    // all loads of a round in flight together
-    const int cap = fdm_split_cap(nx, ny);
-    const int nsx = nx * nx <= cap ? nx * nx : 0;
-    const int nsy = nsx + ny * ny <= cap ? ny * ny : 0;
-    lds_fill3(
-        a, P, [&](int e) { return (double)src[e]; }, vs, nsx, [&](int e) { return Vx[e]; }, vs + nsx, nsy,
-        [&](int e) { return Vy[e]; });
-    const double* vx = nsx ? vs : Vx;
-    const double* vy = nsy ? vs + nsx : Vy;
-    __syncthreads();
-    for (int e = threadIdx.x; e < ny * nc; e += blockDim.x) {
-        const int q = e / nc, il = e - q * nc, i = i0 + il;
-        double acc = 0.0;
-#pragma unroll 8
-        for (int p = 0; p < nx; ++p) acc += vx[p * nx + i] * a[q * nx + p];
-        t[q * cw + il] = acc;
+    const int gx = (nx + 15) >> 4, K = blockIdx.x / gx, i0 = (blockIdx.x - K * gx) * 16;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4, gy = (ny + 15) >> 4;
+    const int ic = imin(i0 + r, nx - 1);
+    const Tin* src = in + (int64_t)K * nx * ny;
+    double* dst = out + (int64_t)K * nx * ny;
+    for (int jt = w; jt < gy; jt += kFdm3Threads / 64) {
+        const int jc = imin(jt * 16 + r, ny - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, nx, [&](int q) { return (double)src[jc * nx + q]; }, [&](int q) { return Vx[q * nx + ic]; },
+                     acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) fdm_lds[(jt * 16 + 4 * v + h) * kFdm3P + r] = acc[v];
     }
     __syncthreads();
-    double* dst = out + (int64_t)K * P;
-    for (int e = threadIdx.x; e < ny * nc; e += blockDim.x) {
-        const int j = e / nc, il = e - j * nc, i = i0 + il;
-        double acc = 0.0;
-#pragma unroll 8
-        for (int q = 0; q < ny; ++q) acc += vy[q * ny + j] * t[q * cw + il];
-        dst[j * nx + i] = acc;
-    }
-}
-
-// row j, columns [i0, i0 + nc): z forward, divide by s*(lx+ly+lz) (0 on the
-// null space), z inverse, in place on data (double)
-__global__ __launch_bounds__(kFdmSplitThreads) void k_fdm_z_cols(int nx, int ny, int nz, double* data,
-                                                                 const double* Vz, const double* lx,
-                                                                 const double* ly, const double* lz, double s,
-                                                                 double eps, const SolverState* st) {
-    if (st->done) return;
-    extern __shared__ double fdm_lds[];
-    const int cw = fdm_split_w(nz), ncb = (nx + cw - 1) / cw;
-    const int j = blockIdx.x / ncb, i0 = (blockIdx.x - j * ncb) * cw;
-    const int nc = imin(cw, nx - i0);
-    const int64_t zs = (int64_t)nx * ny;
-    double* sl = fdm_lds;    // sl[k * cw + il]
-    double* u = sl + nz * cw;
-    double* vs = u + nz * cw;
-    // the column block and the basis (when it fits) in one round of loads
-    const bool sz = nz * nz <= fdm_split_cap(nz, 0);
-    lds_fill2<1, 8>(
-        sl, nz * cw,
-        [&](int e) {
-            const int k = e / cw, il = e - k * cw;
-            return data[k * zs + (int64_t)j * nx + i0 + imin(il, nc - 1)];
-        },
-        vs, sz ? nz * nz : 0, [&](int e) { return Vz[e]; });
-    const double* vz = sz ? vs : Vz;
-    __syncthreads();
-    for (int e = threadIdx.x; e < nz * nc; e += blockDim.x) {
-        const int k = e / nc, il = e - k * nc, i = i0 + il;
-        double acc = 0.0;
-#pragma unroll 8
-        for (int q = 0; q < nz; ++q) acc += vz[q * nz + k] * sl[q * cw + il];
-        const double lam = lx[i] + ly[j] + lz[k];
-        u[k * cw + il] = lam > eps ? acc / (s * lam) : 0.0;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < nz * nc; e += blockDim.x) {
-        const int k = e / nc, il = e - k * nc;
-        double acc = 0.0;
-#pragma unroll 8
-        for (int q = 0; q < nz; ++q) acc += vz[k * nz + q] * u[q * cw + il];
-        data[k * zs + (int64_t)j * nx + i0 + il] = acc;
-    }
-}
-
-// inverse y then x of plane K, rows [j0, j0 + nr): in (double) -> out
-template <typename Tout>
-__global__ __launch_bounds__(kFdmSplitThreads) void k_fdm_inv_rows(int nx, int ny, const double* in, Tout* out,
-                                                                   const double* Vx, const double* Vy,
-                                                                   const SolverState* st) {
-    if (st->done) return;
-    extern __shared__ double fdm_lds[];
-    const int rw = fdm_split_w(nx), nrb = (ny + rw - 1) / rw;
-    const int K = blockIdx.x / nrb, j0 = (blockIdx.x - K * nrb) * rw;
-    const int nr = imin(rw, ny - j0), P = nx * ny;
-    double* a = fdm_lds;   // the plane
-    double* u = a + P;     // its inverse y transform, rows j0.. : u[jl * nx + i]
-    double* vs = u + rw * nx;
-    const double* src = in + (int64_t)K * P;
-    // the plane, Vy and the transpose W[q*nx+i] = Vx[i*nx+q] when they fit
-    // (fdm_split_cap), all loads of a round in flight together
-    const int cap = fdm_split_cap(ny, nx);
-    const int nsy = ny * ny <= cap ? ny * ny : 0;
-    const int nsw = nsy + nx * nx <= cap ? nx * nx : 0;
-    lds_fill3(
-        a, P, [&](int e) { return src[e]; }, vs, nsy, [&](int e) { return Vy[e]; }, vs + nsy, nsw,
-        [&](int e) {
-            const int q = e / nx, i = e - q * nx;
-            return Vx[i * nx + q];
-        });
-    const double* vy = nsy ? vs : Vy;
-    const double* wx = nsw ? vs + nsy : nullptr;
-    __syncthreads();
-    for (int e = threadIdx.x; e < nr * nx; e += blockDim.x) {
-        const int jl = e / nx, i = e - jl * nx, j = j0 + jl;
-        double acc = 0.0;
-#pragma unroll 8
-        for (int q = 0; q < ny; ++q) acc += vy[j * ny + q] * a[q * nx + i];
-        u[jl * nx + i] = acc;
-    }
-    __syncthreads();
-    Tout* dst = out + (int64_t)K * P;
-    for (int e = threadIdx.x; e < nr * nx; e += blockDim.x) {
-        const int jl = e / nx, i = e - jl * nx;
-        double acc = 0.0;
-        if (wx) {
-#pragma unroll 8
-            for (int q = 0; q < nx; ++q) acc += wx[q * nx + i] * u[jl * nx + q];
-        } else {
-#pragma unroll 8
-            for (int q = 0; q < nx; ++q) acc += Vx[i * nx + q] * u[jl * nx + q];
+    for (int jt = w; jt < gy; jt += kFdm3Threads / 64) {
+        const int jc = imin(jt * 16 + r, ny - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, ny, [&](int q) { return Vy[q * ny + jc]; }, [&](int q) { return fdm_lds[q * kFdm3P + r]; },
+                     acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int j = jt * 16 + 4 * v + h;
+            if (j < ny && i0 + r < nx) dst[j * nx + i0 + r] = acc[v];
         }
-        dst[(j0 + jl) * nx + i] = (Tout)acc;
     }
 }
 
-// Whether the 3D coarsest level takes the split passes (PANO_FDM_SPLIT=0: the
-// one-workgroup-per-plane passes).
+// cells [e0, e0 + 16) of every plane: z forward, divide by s*(lx+ly+lz) (0 on
+// the null space), z inverse, in place on data (double)
+__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_z(int nx, int ny, int nz, double* data, const double* Vz,
+                                                         const double* lx, const double* ly, const double* lz,
+                                                         double s, double eps, const SolverState* st) {
+    if (st->done) return;
+    extern __shared__ double fdm_lds[];
+    const int P = nx * ny, lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4;
+    const int e = blockIdx.x * 16 + r, ec = imin(e, P - 1), gz = (nz + 15) >> 4;
+    const double lxy = lx[ec % nx] + ly[ec / nx];
+    for (int kt = w; kt < gz; kt += kFdm3Threads / 64) {
+        const int kc = imin(kt * 16 + r, nz - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, nz, [&](int q) { return Vz[q * nz + kc]; }, [&](int q) { return data[(int64_t)q * P + ec]; },
+                     acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = kt * 16 + 4 * v + h;
+            const double lam = lxy + lz[imin(k, nz - 1)];
+            fdm_lds[k * kFdm3P + r] = lam > eps ? acc[v] / (s * lam) : 0.0;
+        }
+    }
+    __syncthreads();
+    for (int kt = w; kt < gz; kt += kFdm3Threads / 64) {
+        const int kc = imin(kt * 16 + r, nz - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, nz, [&](int q) { return Vz[kc * nz + q]; }, [&](int q) { return fdm_lds[q * kFdm3P + r]; },
+                     acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int k = kt * 16 + 4 * v + h;
+            if (k < nz && e < P) data[(int64_t)k * P + e] = acc[v];
+        }
+    }
+}
+
+// inverse y then x of plane K, rows [j0, j0 + 16): in (double) -> out
+template <typename Tout>
+__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_inv(int nx, int ny, const double* in, Tout* out,
+                                                           const double* Vx, const double* Vy,
+                                                           const SolverState* st) {
+    if (st->done) return;
+    extern __shared__ double fdm_lds[];
+    const int gy = (ny + 15) >> 4, K = blockIdx.x / gy, j0 = (blockIdx.x - K * gy) * 16, R = fdm3_row(nx);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4, gx = (nx + 15) >> 4;
+    const int jc = imin(j0 + r, ny - 1);
+    const double* src = in + (int64_t)K * nx * ny;
+    Tout* dst = out + (int64_t)K * nx * ny;
+    for (int it = w; it < gx; it += kFdm3Threads / 64) {
+        const int ic = imin(it * 16 + r, nx - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, ny, [&](int q) { return Vy[jc * ny + q]; }, [&](int q) { return src[q * nx + ic]; }, acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) fdm_lds[(4 * v + h) * R + it * 16 + r] = acc[v];
+    }
+    __syncthreads();
+    for (int it = w; it < gx; it += kFdm3Threads / 64) {
+        const int ic = imin(it * 16 + r, nx - 1);
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        mfma_tile<8>(0, nx, [&](int q) { return fdm_lds[r * R + q]; }, [&](int q) { return Vx[ic * nx + q]; }, acc);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int j = j0 + 4 * v + h, i = it * 16 + r;
+            if (j < ny && i < nx) dst[j * nx + i] = (Tout)acc[v];
+        }
+    }
+}
+
+// The whole solve of a level of at most 16 cells per axis in one workgroup:
+// one plane (x, y) or row of planes (z) per wave, the field and the bases in
+// LDS as 16^3 and 16 x 16 entries, zero past the level (no product needs a
+// bound). A wave reads its whole plane before it writes it, so the products run
+// in place. 8^3 12 us in three launches, 5.6 in this one; 16^3 in f64 8.8.
+constexpr int kFdm3One = 16, kFdm3OneThreads = 1024;
+template <typename T>
+__global__ __launch_bounds__(kFdm3OneThreads) void k_fdm3_one(int nx, int ny, int nz, const T* in, T* out,
+                                                              const double* Vx, const double* Vy, const double* Vz,
+                                                              const double* lx, const double* ly, const double* lz,
+                                                              double s, double eps, const SolverState* st) {
+    if (st->done) return;
+    constexpr int N = kFdm3One, R = N + 1, PL = N * R;
+    __shared__ double a[N * PL], vv[3][PL];
+    const int t = threadIdx.x;
+    double f[4];
+    const int i = t & 15, j = (t >> 4) & 15, k0 = t >> 8;  // cells (k0 + 4 u, j, i)
+    const bool in_xy = i < nx && j < ny;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 4 * u;
+        f[u] = in_xy && k < nz ? (double)in[(k * ny + j) * nx + i] : 0.0;
+    }
+    if (k0 < 3) {
+        const int n = k0 == 0 ? nx : k0 == 1 ? ny : nz;
+        const double* V = k0 == 0 ? Vx : k0 == 1 ? Vy : Vz;
+        vv[k0][j * R + i] = i < n && j < n ? V[j * n + i] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[(k0 + 4 * u) * PL + j * R + i] = f[u];
+    __syncthreads();
+    const int w = t >> 6, lane = t & 63, r = lane & 15, h = lane >> 4;
+    // out = A B over q of the wave's 16 x 16 entries at o + row * rs + column
+    auto product = [&](double* o, int rs, auto fa, auto fb) {
+        mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < N; q += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(fa(q + h), fb(q + h), acc, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[(4 * v + h) * rs + r] = acc[v];
+    };
+    double* pk = a + w * PL;  // plane k = w
+    double* pj = a + w * R;   // row j = w of every plane
+    if (w < nz) product(pk, R, [&](int q) { return pk[r * R + q]; }, [&](int q) { return vv[0][q * R + r]; });
+    __syncthreads();
+    if (w < nz) product(pk, R, [&](int q) { return vv[1][q * R + r]; }, [&](int q) { return pk[q * R + r]; });
+    __syncthreads();
+    if (w < ny) product(pj, PL, [&](int q) { return vv[2][q * R + r]; }, [&](int q) { return pj[q * PL + r]; });
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 4 * u;
+        double& x = a[k * PL + j * R + i];
+        const double lam = in_xy && k < nz ? lx[i] + ly[j] + lz[k] : 0.0;
+        x = lam > eps ? x / (s * lam) : 0.0;
+    }
+    __syncthreads();
+    if (w < ny) product(pj, PL, [&](int q) { return vv[2][r * R + q]; }, [&](int q) { return pj[q * PL + r]; });
+    __syncthreads();
+    if (w < nz) product(pk, R, [&](int q) { return vv[1][r * R + q]; }, [&](int q) { return pk[q * R + r]; });
+    __syncthreads();
+    if (w < nz) product(pk, R, [&](int q) { return pk[r * R + q]; }, [&](int q) { return vv[0][r * R + q]; });
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int k = k0 + 4 * u;
+        if (in_xy && k < nz) out[(k * ny + j) * nx + i] = (T)a[k * PL + j * R + i];
+    }
+}
+
+// Whether the 3D coarsest level takes the matrix cores (PANO_FDM_SPLIT=0: the
+// one-workgroup-per-plane passes, where a plane and a slice fit LDS).
 static bool fdm_split_on(const Dims& C) {
     const char* e = getenv("PANO_FDM_SPLIT");
-    return !(e && e[0] == '0') && C.d > 1 && C.w * C.h <= kFdmPlane && C.w * C.d <= kFdmPlane;
+    const bool in_lds = C.w * C.h <= kFdmPlane && C.w * C.d <= kFdmPlane;
+    return !in_lds || (C.d > 1 && !(e && e[0] == '0'));
 }
 
 // 3D f32 with the fused passes on: the restriction into the coarsest level is
@@ -844,7 +824,6 @@ template <typename T, int DIM>
 static pano_status coarse_solve(Ctx* c, MG<T>* m, T* z, const T* r, const SolverState* st) {
     const Dims& C = m->dims[m->levels - 1];
     int nx = C.w, ny = C.h, nz = C.d;
-    int64_t n = (int64_t)nx * ny * nz;
     double s = m->s[m->levels - 1];
     double* t0 = m->fdm_tmp[0];
     double* t1 = m->fdm_tmp[1];
@@ -870,55 +849,38 @@ static pano_status coarse_solve(Ctx* c, MG<T>* m, T* z, const T* r, const Solver
         PANO_HIP(hipGetLastError());
         return PANO_OK;
     }
-    if (DIM == 3 && m->fdm_split) {
-        const unsigned nf = (unsigned)(nz * ((nx + fdm_split_w(ny) - 1) / fdm_split_w(ny)));
-        const unsigned nzb = (unsigned)(ny * ((nx + fdm_split_w(nz) - 1) / fdm_split_w(nz)));
-        const unsigned ni = (unsigned)(nz * ((ny + fdm_split_w(nx) - 1) / fdm_split_w(nx)));
-        hipLaunchKernelGGL((k_fdm_fwd_cols<T>), dim3(nf), dim3(kFdmSplitThreads), fdm_split_lds_fwd(nx, ny), S,
-                           nx, ny, r, t0, Vx, Vy, st);
-        hipLaunchKernelGGL(k_fdm_z_cols, dim3(nzb), dim3(kFdmSplitThreads), fdm_split_lds_z(nz), S, nx, ny, nz, t0,
-                           Vz, lx, ly, lz, s, eps, st);
-        hipLaunchKernelGGL((k_fdm_inv_rows<T>), dim3(ni), dim3(kFdmSplitThreads), fdm_split_lds_inv(nx, ny), S,
-                           nx, ny, (const double*)t0, z, Vx, Vy, st);
-        PANO_HIP(hipGetLastError());
-        return PANO_OK;
-    }
-    if (DIM == 3 && nx * ny <= kFdmPlane && nx * nz <= kFdmPlane) {
-        size_t lds = kFdmLdsBytes;
-        {
-            if constexpr (std::is_same<T, float>::value) {
-                if (coarse_rc<T, DIM>(m))
-                    hipLaunchKernelGGL(k_fdm_plane_rc, dim3(nz), dim3(kFdmThreads), lds, S, m->dims[m->levels - 2],
-                                       C, (const float*)r, t0, Vx, Vy, s, eps, st);
-                else
-                    hipLaunchKernelGGL((k_fdm_plane<T, double>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 0, r,
-                                       t0, Vx, Vy, (const double*)nullptr, (const double*)nullptr, s, eps, st);
-            } else {
-                hipLaunchKernelGGL((k_fdm_plane<T, double>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 0, r, t0,
-                                   Vx, Vy, (const double*)nullptr, (const double*)nullptr, s, eps, st);
-            }
-            hipLaunchKernelGGL(k_fdm_zcol, dim3(ny), dim3(kFdmThreads), lds, S, nx, ny, nz, t0, Vz, lx, ly, lz, s, eps,
-                               st);
-            hipLaunchKernelGGL((k_fdm_plane<double, T>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 1, t0, z, Vx, Vy,
-                               (const double*)nullptr, (const double*)nullptr, s, eps, st);
+    if (m->fdm_split) {
+        if (nx <= kFdm3One && ny <= kFdm3One && nz <= kFdm3One) {
+            hipLaunchKernelGGL((k_fdm3_one<T>), dim3(1), dim3(kFdm3OneThreads), 0, S, nx, ny, nz, r, z, Vx, Vy, Vz, lx,
+                               ly, lz, s, eps, st);
+            PANO_HIP(hipGetLastError());
+            return PANO_OK;
         }
+        const unsigned gx = (unsigned)((nx + 15) / 16), gy = (unsigned)((ny + 15) / 16);
+        hipLaunchKernelGGL((k_fdm3_fwd<T>), dim3(nz * gx), dim3(kFdm3Threads), fdm3_lds_cols(ny), S, nx, ny, r, t0, Vx,
+                           Vy, st);
+        hipLaunchKernelGGL(k_fdm3_z, dim3((nx * ny + 15) / 16), dim3(kFdm3Threads), fdm3_lds_cols(nz), S, nx, ny, nz,
+                           t0, Vz, lx, ly, lz, s, eps, st);
+        hipLaunchKernelGGL((k_fdm3_inv<T>), dim3(nz * gy), dim3(kFdm3Threads),
+                           (size_t)16 * fdm3_row(nx) * sizeof(double), S, nx, ny, (const double*)t0, z, Vx, Vy, st);
         PANO_HIP(hipGetLastError());
         return PANO_OK;
     }
-    // large coarsest planes: one global-memory pass per axis
-    unsigned nb = blocks_for(n, kBlock);
-    hipLaunchKernelGGL((k_fdm_axis<T, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 0, 0, r, t0, Vx, 0,
-                       nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 0, t0, t1, Vy,
-                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 0, t1, t0, Vz,
-                       1, lx, ly, lz, s, eps, st);
-    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 2, 1, t0, t1, Vz,
-                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    hipLaunchKernelGGL((k_fdm_axis<double, double>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 1, 1, t1, t0, Vy,
-                       0, nullptr, nullptr, nullptr, 0.0, 0.0, st);
-    hipLaunchKernelGGL((k_fdm_axis<double, T>), dim3(nb), dim3(kBlock), 0, S, nx, ny, nz, 0, 1, t0, z, Vx, 0,
-                       nullptr, nullptr, nullptr, 0.0, 0.0, st);
+    const size_t lds = kFdmLdsBytes;
+    if constexpr (std::is_same<T, float>::value) {
+        if (coarse_rc<T, DIM>(m))
+            hipLaunchKernelGGL(k_fdm_plane_rc, dim3(nz), dim3(kFdmThreads), lds, S, m->dims[m->levels - 2], C,
+                               (const float*)r, t0, Vx, Vy, s, eps, st);
+        else
+            hipLaunchKernelGGL((k_fdm_plane<T, double>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 0, r, t0, Vx, Vy,
+                               (const double*)nullptr, (const double*)nullptr, s, eps, st);
+    } else {
+        hipLaunchKernelGGL((k_fdm_plane<T, double>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 0, r, t0, Vx, Vy,
+                           (const double*)nullptr, (const double*)nullptr, s, eps, st);
+    }
+    hipLaunchKernelGGL(k_fdm_zcol, dim3(ny), dim3(kFdmThreads), lds, S, nx, ny, nz, t0, Vz, lx, ly, lz, s, eps, st);
+    hipLaunchKernelGGL((k_fdm_plane<double, T>), dim3(nz), dim3(kFdmThreads), lds, S, nx, ny, 1, t0, z, Vx, Vy,
+                       (const double*)nullptr, (const double*)nullptr, s, eps, st);
     PANO_HIP(hipGetLastError());
     return PANO_OK;
 }

@@ -588,70 +588,6 @@ __device__ __forceinline__ void lds_fill(double* dst, int n, Src src) {
     }
 }
 
-// Three fills at once (n0, n1, n2 >= 0): each round issues a thread's loads
-// of all three before it stores any, so a workgroup staging a plane and two
-// bases waits for one memory round trip, not three. The loads are
-// unconditional (a branch per load would wait for each one): a source must
-// be readable at index 0 also when its segment is empty, which then stores
-// nothing.
-template <typename S0, typename S1, typename S2>
-__device__ __forceinline__ void lds_fill3(double* d0, int n0, S0 s0, double* d1, int n1, S1 s1, double* d2, int n2,
-                                          S2 s2) {
-    constexpr int U = 8;
-    const int nm = n0 > n1 ? (n0 > n2 ? n0 : n2) : (n1 > n2 ? n1 : n2);
-    const int c0 = n0 > 0 ? n0 - 1 : 0, c1 = n1 > 0 ? n1 - 1 : 0, c2 = n2 > 0 ? n2 - 1 : 0;
-    for (int base = threadIdx.x; base < nm; base += U * blockDim.x) {
-        double v0[U], v1[U], v2[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = base + u * blockDim.x;
-            v0[u] = s0(e < c0 ? e : c0);
-            v1[u] = s1(e < c1 ? e : c1);
-            v2[u] = s2(e < c2 ? e : c2);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = base + u * blockDim.x;
-            if (e < n0) d0[e] = v0[u];
-            if (e < n1) d1[e] = v1[u];
-            if (e < n2) d2[e] = v2[u];
-        }
-    }
-}
-
-// Two fills at once with U0 / U1 loads per thread and round: a thread issues
-// all its loads of a round before it stores any, so with enough loads per
-// round (a staged basis of up to U1 * blockDim.x doubles) a workgroup waits
-// for one memory round trip. Unconditional loads as in lds_fill3.
-template <int U0, int U1, typename S0, typename S1>
-__device__ __forceinline__ void lds_fill2(double* d0, int n0, S0 s0, double* d1, int n1, S1 s1) {
-    const int B = blockDim.x;
-    const int c0 = n0 > 0 ? n0 - 1 : 0, c1 = n1 > 0 ? n1 - 1 : 0;
-    for (int r0 = threadIdx.x, r1 = threadIdx.x; r0 < n0 || r1 < n1; r0 += U0 * B, r1 += U1 * B) {
-        double v0[U0], v1[U1];
-#pragma unroll
-        for (int u = 0; u < U0; ++u) {
-            const int e = r0 + u * B;
-            v0[u] = s0(e < c0 ? e : c0);
-        }
-#pragma unroll
-        for (int u = 0; u < U1; ++u) {
-            const int e = r1 + u * B;
-            v1[u] = s1(e < c1 ? e : c1);
-        }
-#pragma unroll
-        for (int u = 0; u < U0; ++u) {
-            const int e = r0 + u * B;
-            if (e < n0) d0[e] = v0[u];
-        }
-#pragma unroll
-        for (int u = 0; u < U1; ++u) {
-            const int e = r1 + u * B;
-            if (e < n1) d1[e] = v1[u];
-        }
-    }
-}
-
 __device__ __forceinline__ const double* stage_basis(double* dst, int used, const double* V, int n) {
     if (used + n * n > kFdmVStage) return V;
     lds_fill(dst + used, n * n, [&](int e) { return V[e]; });
@@ -699,7 +635,7 @@ __device__ __forceinline__ void lds_axis_r(const double* a, double* b, int nx, i
             for (int q = 0; q < n; ++q) {
                 const double w = V[wb + q * ws];
 #pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] += w * a[jr[r] * nx + q];
+                for (int r = 0; r < R; ++r) acc[r] = __builtin_fma(w, a[jr[r] * nx + q], acc[r]);
             }
         } else {
             // out[j][i] = sum_q W(q, j) a[q][i], W(q, j) = V[q*ny+j] (forward) or V[j*ny+q] (inverse)
@@ -708,7 +644,7 @@ __device__ __forceinline__ void lds_axis_r(const double* a, double* b, int nx, i
             for (int q = 0; q < n; ++q) {
                 const double v = a[q * nx + i];
 #pragma unroll
-                for (int r = 0; r < R; ++r) acc[r] += V[(inverse ? jr[r] * ny : jr[r]) + q * ws] * v;
+                for (int r = 0; r < R; ++r) acc[r] = __builtin_fma(V[(inverse ? jr[r] * ny : jr[r]) + q * ws], v, acc[r]);
             }
         }
 #pragma unroll
