@@ -114,12 +114,42 @@ __global__ __launch_bounds__(256) void k_neg_div(Dims D, Grid3 G, T* b, Faces<co
         if (z0 + k < D.d) stx(b, cell_index(D, z0 + k, y, x), out[k]);
 }
 
+// q = A p. In 3D runs of planes, as the divergence: a thread per cell waited
+// for its seven loads and shared none (125 x 131 x 193 f32: 15.8 us, 8.7 in runs).
 template <typename T, int DIM>
 __global__ __launch_bounds__(256) void k_poisson(Dims D, Grid3 G, T* q, const T* p, T dt) {
-    int x, y, z, L;
-    tile_xyz(G, x, y, z, L);
+    constexpr int NZ = kPlaneRun<DIM>;
+    int x, y, zb, L;
+    tile_xyz(G, x, y, zb, L);
     if (x >= D.w || y >= D.h) return;
-    q[cell_index(D, z, y, x)] = poisson_value<T, DIM, NATURAL>(D, p, dt, z, y, x);
+    if constexpr (DIM == 2) {
+        q[cell_index(D, 0, y, x)] = poisson_value<T, DIM, NATURAL>(D, p, dt, 0, y, x);
+    } else {
+        // every load of the run first; a missing neighbour reads a cell that is
+        // there and poisson_from ignores it
+        const int z0 = zb * NZ;
+        const int dl = x > 0, dr = x < D.w - 1, dy = y > 0 ? D.w : 0, db = y < D.h - 1 ? D.w : 0;
+        T c[NZ + 2], xl[NZ], xr[NZ], yl[NZ], yr[NZ];
+#pragma unroll
+        for (int k = 0; k < NZ + 2; ++k)
+            c[k] = ldx(p, (int)cell_index(D, imin(imax(z0 + k - 1, 0), D.d - 1), y, x));
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            const int i = (int)cell_index(D, imin(z0 + k, D.d - 1), y, x);
+            xl[k] = ldx(p, i - dl);
+            xr[k] = ldx(p, i + dr);
+            yl[k] = ldx(p, i - dy);
+            yr[k] = ldx(p, i + db);
+        }
+#pragma unroll
+        for (int k = 0; k < NZ; ++k) {
+            const int z = z0 + k;
+            if (z >= D.d) continue;
+            stx(q, (int)cell_index(D, z, y, x),
+                poisson_from<T, DIM>(c[k + 1], xl[k], xr[k], yl[k], yr[k], c[k], c[k + 2],
+                                     nbr_bits<DIM>(D, z, y, x), D.bc, dt));
+        }
+    }
 }
 
 // The literal closure with the reference's obstacle mask (dec_fluid.rs:104-112):
@@ -315,7 +345,8 @@ pano_status launch_poisson_apply(Ctx* c, const Dims& D, double dt, const uint8_t
             return fail(PANO_ERR_BAD_SHAPE, "face_mask needs a 2D grid with closed walls");
         LAUNCH3((k_poisson_masked2<T>), G, D, G, q, p, (T)dt, mask);
     } else if (D.d > 1) {
-        LAUNCH3((k_poisson<T, 3>), G, D, G, q, p, (T)dt);
+        const Grid3 Gr = grid3_run(D.w, D.h, D.d, kPlaneRun<3>);
+        LAUNCH3((k_poisson<T, 3>), Gr, D, Gr, q, p, (T)dt);
     } else {
         LAUNCH3((k_poisson<T, 2>), G, D, G, q, p, (T)dt);
     }
