@@ -21,7 +21,7 @@ struct MG {
     double* fdm_lam[3] = {nullptr, nullptr, nullptr};   // eigenvalues
     int coarse_n[3] = {1, 1, 1};                         // coarsest extents x, y, z
     bool tb = true;  // 3D f32 levels: pre/post-smoothing as one pass each (PANO_MG_FUSED=0 turns it off)
-    bool fdm_split = false;  // 3D coarsest level: passes split over many workgroups (PANO_FDM_SPLIT=0: off)
+    bool fdm_split = false;  // 3D coarsest level on the matrix cores (fdm_split_on)
     // levels above the coarsest that smooth in one pass or run their legs as
     // one launch each: the prolongation runs inside the post-smoothing
     // (PANO_MG_PRO=0: off), which then reads the pre-smoothed z from w[l]
