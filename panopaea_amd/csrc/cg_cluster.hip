@@ -20,9 +20,10 @@
 // turn), all written by every workgroup: readers of one address wait for each
 // other (128^2: 5.8 us per iteration with one mailbox, 4.7 with 8, 4.6 with 32).
 // Copies: two of hb, z.r and max|r|, four of p.q. Once the p.q exchange of
-// iteration k is over, everybody has left iteration k - 1, so its copies are
-// emptied there; those stores have completed (s_waitcnt) before the
-// workgroup's next p.q is stored, which everybody waits for before a copy
+// iteration k is over for a whole workgroup (behind the barrier after the
+// poll: each wave polls 64 slots only), everybody has left iteration k - 1, so
+// its copies are emptied there; those stores have completed (s_waitcnt) before
+// the workgroup's next p.q is stored, which everybody waits for before a copy
 // emptied here is polled again.
 //
 // Sums are FP64 as in the launches' partials, in another order. Everything
@@ -275,14 +276,15 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
         bool got = cl_poll<1>(S[mr].pq[k4], nullptr, &S->stop, P, spin, v);
         s = wave_all<ClSum>(v[0]);
         if ((t & 63) == 0) red[1][0][wave] = s;
+        if (!got) flag = 0;
+        __syncthreads();
+        if (!flag) break;
+        // only now have the waves together seen every p.q: a wave has seen its own slots'
         if (t < kClCopies) {
             st_agent(&S[t].pq[(k + 3) & 3][g], kClEmpty);
             st_agent(&S[t].zr[k2 ^ 1][g], kClEmpty);
             st_agent(&S[t].mx[k2 ^ 1][g], kClEmpty);
         }
-        if (!got) flag = 0;
-        __syncthreads();
-        if (!flag) break;
         pq = waves_all<ClSum, NW>(red[1][0]);
         alpha = sigma / pq;
         if (!(alpha == alpha) || fabs(alpha) > 1.7e308) {
