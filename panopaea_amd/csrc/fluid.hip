@@ -114,11 +114,10 @@ __global__ __launch_bounds__(256) void k_neg_div(Dims D, Grid3 G, T* b, Faces<co
         if (z0 + k < D.d) stx(b, cell_index(D, z0 + k, y, x), out[k]);
 }
 
-// q = A p. In 3D runs of planes, as the divergence: a thread per cell waited
+// q = A p. In 3D runs of NZ planes, as the divergence: a thread per cell waited
 // for its seven loads and shared none (125 x 131 x 193 f32: 15.8 us, 8.7 in runs).
-template <typename T, int DIM>
+template <typename T, int DIM, int NZ>
 __global__ __launch_bounds__(256) void k_poisson(Dims D, Grid3 G, T* q, const T* p, T dt) {
-    constexpr int NZ = kPlaneRun<DIM>;
     int x, y, zb, L;
     tile_xyz(G, x, y, zb, L);
     if (x >= D.w || y >= D.h) return;
@@ -336,6 +335,18 @@ static pano_status launch_neg_div_masked(Ctx* c, const Dims& D, T* b, const T* f
     return PANO_OK;
 }
 
+// The planes per thread of the 3D operator: runs save loads, but they are
+// longer chains in fewer waves, which small fields wait for. Kernel time in us
+// with runs of 1 / 2 / 4, by the tiles of single planes:
+//   f32  576 (48^3)  2.76 / 2.80 / 2.96   1024 (64^3)  3.04 / 2.92 / 2.92   1232 (44x56x76)  3.20 / 3.20 / 3.12
+//   f64 1024 (64^3)  3.40 / 3.44 / 3.56   2040 (136x57x20)  4.32 / 4.12 / 4.12   3200 (16x200x200)  5.92 / 5.92 / 6.60
+//       8192 (128^3) 10.6 / 9.44 / 9.40  16500 (125x131x193)  17.4 / 16.0 / 15.9  40000 (200^3)  37.6 / 33.6 / 31.9
+template <typename T>
+static int poisson_run(const Grid3& one) {
+    if (sizeof(T) == 4) return one.nb < 1024 ? 1 : 4;
+    return one.nb < 2048 ? 1 : one.nb < 16384 ? 2 : 4;
+}
+
 template <typename T>
 pano_status launch_poisson_apply(Ctx* c, const Dims& D, double dt, const uint8_t* mask, T* q,
                                  const T* p) {
@@ -345,10 +356,13 @@ pano_status launch_poisson_apply(Ctx* c, const Dims& D, double dt, const uint8_t
             return fail(PANO_ERR_BAD_SHAPE, "face_mask needs a 2D grid with closed walls");
         LAUNCH3((k_poisson_masked2<T>), G, D, G, q, p, (T)dt, mask);
     } else if (D.d > 1) {
-        const Grid3 Gr = grid3_run(D.w, D.h, D.d, kPlaneRun<3>);
-        LAUNCH3((k_poisson<T, 3>), Gr, D, Gr, q, p, (T)dt);
+        const int nz = poisson_run<T>(G);
+        const Grid3 Gr = grid3_run(D.w, D.h, D.d, nz);
+        if (nz == 1) LAUNCH3((k_poisson<T, 3, 1>), Gr, D, Gr, q, p, (T)dt);
+        else if (nz == 2) LAUNCH3((k_poisson<T, 3, 2>), Gr, D, Gr, q, p, (T)dt);
+        else LAUNCH3((k_poisson<T, 3, 4>), Gr, D, Gr, q, p, (T)dt);
     } else {
-        LAUNCH3((k_poisson<T, 2>), G, D, G, q, p, (T)dt);
+        LAUNCH3((k_poisson<T, 2, 1>), G, D, G, q, p, (T)dt);
     }
     return PANO_OK;
 }
