@@ -250,6 +250,9 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
 
     double sigma = s0.sigma, alpha = s0.alpha, beta = s0.beta, pq = s0.pq, rnorm = s0.rnorm;
     int iter = s0.iter, conv = 0, bad = 0;
+    // the thread's halo polls behind the exchange's barrier were answered: told
+    // at the next exchange, as slower waves may still have to read `flag`
+    bool kept = true;
     for (int k = 0; iter < s0.max_iter; ++k) {
         const int k2 = k & 1, k4 = k & 3;
         T* hb = k2 ? hb1 : hb0;
@@ -276,7 +279,7 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
         bool got = cl_poll<1>(S[mr].pq[k4], nullptr, &S->stop, P, spin, v);
         s = wave_all<ClSum>(v[0]);
         if ((t & 63) == 0) red[1][0][wave] = s;
-        if (!got) flag = 0;
+        if (!got || !kept) flag = 0;
         __syncthreads();
         if (!flag) break;
         // only now have the waves together seen every p.q: a wave has seen its own slots'
@@ -392,7 +395,7 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
                 zh[c] = (T)((double)cl_z<T, JAC>(hz[C + c], ncz[c] >> 8, dt) + beta * (double)zh[c]);
             }
         }
-        if (!got) flag = 0;  // seen at the next exchange
+        kept = got;
         __syncthreads();
     }
     if (!flag) {  // abandoned (uniform): the host starts over with the launches

@@ -5,7 +5,8 @@
 // wave waits for them), and one wave of one workgroup is held back while all
 // others go on as far as they can. Whatever the order, the loop has to reach
 // its end without a wait running out and give the same bits, for clusters of
-// more workgroups than a wave has lanes above all.
+// more workgroups than a wave has lanes above all; and where waits run out (a
+// few polls allowed only), the waves of a workgroup have to leave together.
 #include <sched.h>
 #include <semaphore.h>
 #include <setjmp.h>
@@ -39,7 +40,15 @@ struct Store {
     char* p;
     unsigned char v[8];
     size_t n;
+    long due;  // turns of all waves before which it does not arrive by itself
 };
+long g_turns;
+// Late: edge values in these bytes arrive after `turns` only, and wave `wave` of
+// workgroup `wg` leaves its `barrier`-th barrier as late.
+struct Late {
+    const char *lo = nullptr, *hi = nullptr;
+    int wg = -1, wave = 0, barrier = 0, turns = 0;
+} g_late;
 long g_stores;  // that have reached memory
 struct Wave {
     Lane st[64];
@@ -49,17 +58,20 @@ struct Wave {
     std::vector<Store> pending;
     bool done = false, bar = false;
     int polls = 0;   // scheduling points passed
+    int barriers = 0;
+    long held = 0;   // turn of all waves up to which this one is held
     int same = 0;    // of them the last ones with no store to memory since
     long seen = -1;
-    void flush_one(size_t i) {
-        ++g_stores;
+    void flush_one(size_t i, bool wait = false) {
         for (size_t j = 0; j < i; ++j)  // stores to one address stay in order
             if (pending[j].p == pending[i].p) { i = j; break; }
+        if (!wait && g_turns < pending[i].due) return;
+        ++g_stores;
         memcpy(pending[i].p, pending[i].v, pending[i].n);
         pending.erase(pending.begin() + i);
     }
     void flush() {
-        while (!pending.empty()) flush_one(rnd((unsigned)pending.size()));
+        while (!pending.empty()) flush_one(rnd((unsigned)pending.size()), true);
     }
 };
 constexpr size_t kStack = 24 << 10;
@@ -159,6 +171,8 @@ void step(Group* g, int wave) {
             if (!v.bar) continue;
             v.bar = false;
             v.same = 0;
+            if (g->id == g_late.wg && &v == &g->w[g_late.wave] && ++v.barriers == g_late.barrier)
+                v.held = g_turns + g_late.turns;
             for (int l = 0; l < 64; ++l)
                 if (v.st[l] == BAR) v.st[l] = RUN;
         }
@@ -173,11 +187,13 @@ int collective(int op, int v) {
     return t_w->out[t_lane];
 }
 
-// A wave that polls memory nobody has written to since is left out: kIdle polls are more than any loop's loads per try.
+// A wave that polls memory nobody has written to since is left out (unless
+// waits are to run out): kIdle polls are more than any loop's loads per try.
 // Once that holds for every wave, nothing will ever end the waits.
 constexpr int kIdle = 8;
+bool g_skip_idle = true;
 
-// The wave to hold back: from its scheduling point `at` on, for `steps` steps of the others.
+// The wave to hold back: from its scheduling point `at` on, for `steps` of its turns.
 struct Hold {
     int wg = -1, wave = 0, at = 0, steps = 0;
 } g_hold;
@@ -190,7 +206,7 @@ int emu_dpp(int, int v, int ctrl, int, int, bool) { return collective(ctrl, v); 
 int emu_readlane(int v, int lane) { return collective(2000 + lane, v); }
 void emu_waitcnt() { t_w->flush(); }
 void emu_store(void* p, const void* v, size_t n) {
-    Store s{(char*)p, {}, n};
+    Store s{(char*)p, {}, n, p >= g_late.lo && p < g_late.hi ? g_turns + g_late.turns : 0};
     memcpy(s.v, v, n);
     t_w->pending.push_back(s);
 }
@@ -247,6 +263,7 @@ bool emu_launch(dim3 grid, dim3 block, size_t lds, void (*body)(void*), void* ar
             _exit(1);
         }
         const unsigned i = rnd((unsigned)open.size());
+        ++g_turns;
         Group* g = gs[open[i].first].get();
         const int k = open[i].second;
         Wave& w = g->w[k];
@@ -255,6 +272,10 @@ bool emu_launch(dim3 grid, dim3 block, size_t lds, void (*body)(void*), void* ar
             while (!w.pending.empty() && rnd(8)) w.flush_one(rnd((unsigned)w.pending.size()));
         }
         if (w.bar) continue;
+        if (g_turns < w.held) {
+            idle = 0;
+            continue;
+        }
         if (g->id == h.wg && k == h.wave && w.polls >= h.at && h.steps > 0) {
             --h.steps;
             idle = 0;
@@ -262,7 +283,7 @@ bool emu_launch(dim3 grid, dim3 block, size_t lds, void (*body)(void*), void* ar
         }
         w.same = w.seen == g_stores ? w.same + 1 : 0;
         w.seen = g_stores;
-        if (w.same > kIdle) continue;
+        if (g_skip_idle && w.same > kIdle) continue;
         idle = 0;
         ++w.polls;
         g->pick = k;
@@ -320,6 +341,9 @@ static Run<T> solve(const Dims& D, int chunk, bool jacobi, int iterations, unsig
     P.wgs = (n + chunk - 1) / chunk;
     P.lds = (size_t)(chunk + 2 * D.w) * sizeof(T) + 2 * D.w;
     static ClSlots slots[kClCopies];
+    const int behind = (g_late.wg + 1) * chunk;
+    g_late.lo = g_late.wg < 0 ? nullptr : (const char*)(hb.data() + behind);
+    g_late.hi = g_late.wg < 0 ? nullptr : (const char*)(hb.data() + (behind + 100 < n ? behind + 100 : n));
     Ctx c;
     cl_solve<T>(&c, D, P, jacobi, R.x.data(), R.r.data(), p.data(), hb.data(), dt, nullptr, &R.st, slots, spin);
     return R;
@@ -358,6 +382,36 @@ static void orders(const char* what, const Dims& D, int chunk, bool jacobi, int 
     }
 }
 
+// Waits run out after `spin` polls: an abandoned run says so, and no wave waits
+// at a barrier for one that has left.
+template <typename T>
+static void abandoned(const char* what, const Dims& D, int chunk, int iterations, int seeds) {
+    g_skip_idle = false;
+    g_hold = Hold();
+    int stalls = 0;
+    for (int s = 0; s < seeds; ++s) {
+        g_rng.seed(1000 + s);
+        g_divergent = false;
+        const unsigned spin = 30 + rnd(120);
+        // the first cells behind a workgroup's own, which long rows poll behind the exchange's barrier
+        g_late.wg = (int)rnd(D.d * D.h * D.w / chunk - 1);
+        g_late.wave = (int)rnd(4);
+        g_late.barrier = 1 + (int)rnd(6);
+        g_late.turns = 30000;
+        const Run<T> R = solve<T>(D, chunk, true, iterations, spin);
+        ++runs;
+        stalls += R.st.stalled != 0;
+        if (g_divergent || !(R.st.stalled || (R.st.done && R.st.iter == iterations))) {
+            ++fails;
+            printf("FAIL %s, order %d, %u polls: %s stalled %d done %d\n", what, s, spin,
+                   g_divergent ? "a wave left its workgroup's others at a barrier" : "", R.st.stalled, R.st.done);
+        }
+    }
+    printf("%s: %d of %d runs abandoned\n", what, stalls, seeds);
+    g_skip_idle = true;
+    g_late = Late();
+}
+
 int main() {
     cpu_set_t one;  // one thread runs at a time
     CPU_ZERO(&one);
@@ -368,6 +422,7 @@ int main() {
     orders<double>("3D Jacobi", Dims{17, 16, 17, 32}, 64, true, 4, 4);
     orders<double>("2D identity", Dims{1, 130, 64, 2}, 64, false, 3, 3);
     orders<float>("2D identity", Dims{1, 256, 64, 0}, 64, false, 2, 1);
+    abandoned<float>("few workgroups, long rows", Dims{1, 3, 300, 0}, 64, 3, 100);
     printf("%d orders, %d failures\n", runs, fails);
     return fails != 0;
 }
