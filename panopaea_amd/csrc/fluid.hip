@@ -256,8 +256,9 @@ pano_status launch_advect(Ctx* c, const Dims& D, T* dst, const T* src, double dt
 }
 
 bool advect_fused_on(const Dims& D) {
+    if (D.d <= 1) return false;
     const char* e = getenv("PANO_ADV_FUSED");
-    return D.d > 1 && !(e && e[0] == '0');
+    return !(e && e[0] == '0');
 }
 
 // The one-pass advection's launch. Tiles of 32 x 16 cells (256^3 faces 211 us
