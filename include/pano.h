@@ -173,6 +173,16 @@ pano_status pano_precond_conjugate_gradient(pano_ctx, const pano_grid*, const pa
                                             void* x, const void* b, void* residual,
                                             void* auxiliary, void* search, pano_pcg_info* info);
 
+/* No reference counterpart. Identity and Jacobi solves (and steps) of small
+ * grids run their CG loop as one kernel whose workgroups wait for each other;
+ * where they do not all get to run (the device is shared), the kernel gives up
+ * and the solve runs again as separate launches. Counts of this context: the
+ * solves begun that way and those of them given up (either pointer may be
+ * null). The launches are also taken while a kernel timer runs and with
+ * PANO_CG_CLUSTER=0 in the environment; with PANO_CG_CLUSTER=1 a wait is given
+ * up at once. */
+pano_status pano_cg_cluster_counts(pano_ctx ctx, int64_t* solves, int64_t* abandoned);
+
 /* No reference counterpart: pano_precond_conjugate_gradient for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). Same arguments, arithmetic and results

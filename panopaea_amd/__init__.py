@@ -52,6 +52,13 @@ class Context:
     def stream(self):
         return _lib.lib().pano_ctx_stream(self.handle)
 
+    def cluster_counts(self):
+        """(solves whose CG loop was begun as one kernel, those of them that were
+        given up and run again as launches)."""
+        n, a = ctypes.c_int64(), ctypes.c_int64()
+        _lib.check(_lib.lib().pano_cg_cluster_counts(self.handle, ctypes.byref(n), ctypes.byref(a)))
+        return n.value, a.value
+
     def close(self):
         if self.handle:
             _lib.lib().pano_ctx_destroy(self.handle)

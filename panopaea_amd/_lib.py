@@ -109,6 +109,7 @@ _SIGS = {
     "pano_memcpy_htod": ([c_void_p, c_void_p, c_void_p, ctypes.c_size_t], c_i32),
     "pano_memcpy_dtoh": ([c_void_p, c_void_p, c_void_p, ctypes.c_size_t], c_i32),
     "pano_fill_zero": ([c_void_p, c_void_p, ctypes.c_size_t], c_i32),
+    "pano_cg_cluster_counts": ([c_void_p, _P(c_i64), _P(c_i64)], c_i32),
     "pano_timer_start": ([c_void_p, ctypes.c_char_p], c_i32),
     "pano_timer_stop": ([c_void_p, _P(c_f64), _P(c_i64), _P(c_f64)], c_i32),
     "pano_num_elem_0": ([_P(GridDesc)], c_i64),

@@ -91,6 +91,7 @@ struct Ctx {
     SolverState* host_state = nullptr;   // pinned mirror of the device state
     hipEvent_t ev[2] = {nullptr, nullptr};
     int num_cu = 256;
+    int64_t cl_solves = 0, cl_abandoned = 0;  // one-kernel CG loops begun, and given up
     // While `arena` is set (by the no-allocation entry point, for one call),
     // workspace() hands out consecutive 256-byte aligned ranges of it instead
     // of pooled allocations, and fails once `arena_cap` would be exceeded.

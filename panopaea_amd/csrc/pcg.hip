@@ -500,7 +500,9 @@ static pano_status solver_run(Solver<T>* S, int max_iterations, int every, const
         PANO_HIP(hipMemcpyAsync(&c->host_state[0], S->st, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
         PANO_HIP(hipStreamSynchronize(c->stream));
         c->timer.solve = -1;
+        c->cl_solves += 1;
         if (!c->host_state[0].stalled) return PANO_OK;
+        c->cl_abandoned += 1;
         PANO_CHECK(start());
     }
     return solver_loop<T>(S, max_iterations, every, key, epi);
@@ -917,6 +919,14 @@ pano_status pano_precond_conjugate_gradient(pano_ctx ctx, const pano_grid* g, co
                                  (double*)search, info, false);
     return pcg_solve<float>(c, D, P, (float*)x, (const float*)b, (float*)residual, (float*)auxiliary,
                             (float*)search, info, false);
+}
+
+pano_status pano_cg_cluster_counts(pano_ctx ctx, int64_t* solves, int64_t* abandoned) {
+    Ctx* c = ctx_of(ctx);
+    if (!c) return fail(PANO_ERR_INVALID, "ctx is null");
+    if (solves) *solves = c->cl_solves;
+    if (abandoned) *abandoned = c->cl_abandoned;
+    return PANO_OK;
 }
 
 pano_status pano_precond_apply(pano_ctx ctx, const pano_grid* g, const pano_pcg_params* P, void* dst,
