@@ -178,7 +178,9 @@ pano_status pano_precond_conjugate_gradient(pano_ctx, const pano_grid*, const pa
  * where they do not all get to run (the device is shared), the kernel gives up
  * and the solve runs again as separate launches. Counts of this context: the
  * solves begun that way and those of them given up (either pointer may be
- * null). The launches are also taken while a kernel timer runs and with
+ * null). After two in a row that were given up the next solve takes the
+ * launches at once, after three the next three, and so on up to 1023, until one
+ * ends. The launches are also taken while a kernel timer runs and with
  * PANO_CG_CLUSTER=0 in the environment; with PANO_CG_CLUSTER=1 a wait is given
  * up at once. */
 pano_status pano_cg_cluster_counts(pano_ctx ctx, int64_t* solves, int64_t* abandoned);

@@ -81,6 +81,32 @@ struct KernelTimer {
     double bytes = 0.0;               // algorithmic bytes per launch (set by the kernel site)
 };
 
+// One-kernel CG loops of a context: those begun, those given up, and when to
+// stay with the launches. A loop gives up after a quarter of a second of waits,
+// because something else holds the device's CUs; that may be so for long, and
+// then every solve would pay for it. So after the second one in a row the next
+// solve takes the launches, after the third the next three, then 7, ... 1023;
+// one that ends sets this back.
+struct ClusterUse {
+    int64_t solves = 0, abandoned = 0;
+    int in_a_row = 0, skip = 0;
+    bool take() {
+        if (skip == 0) return true;
+        --skip;
+        return false;
+    }
+    void ended(bool gave_up) {
+        solves += 1;
+        if (!gave_up) {
+            in_a_row = 0;
+            return;
+        }
+        abandoned += 1;
+        if (in_a_row < 11) in_a_row += 1;
+        skip = (1 << (in_a_row - 1)) - 1;
+    }
+};
+
 struct Ctx {
     int device = 0;
     KernelTimer timer;
@@ -91,7 +117,7 @@ struct Ctx {
     SolverState* host_state = nullptr;   // pinned mirror of the device state
     hipEvent_t ev[2] = {nullptr, nullptr};
     int num_cu = 256;
-    int64_t cl_solves = 0, cl_abandoned = 0;  // one-kernel CG loops begun, and given up
+    ClusterUse cl;
     // While `arena` is set (by the no-allocation entry point, for one call),
     // workspace() hands out consecutive 256-byte aligned ranges of it instead
     // of pooled allocations, and fails once `arena_cap` would be exceeded.

@@ -492,7 +492,7 @@ static pano_status solver_run(Solver<T>* S, int max_iterations, int every, const
                               Epi&& epi) {
     Ctx* c = S->c;
     PANO_CHECK(start());
-    if (S->cl.wgs) {
+    if (S->cl.wgs && c->cl.take()) {
         const ClReserve cus(c->device, S->cl.wgs, c->num_cu);
         PANO_CHECK(cl_solve<T>(c, S->D, S->cl, S->precond == PANO_PRECOND_JACOBI, S->x, S->r, S->p, S->aux, S->dt,
                                S->mask, S->st, S->slots, S->spin));
@@ -500,9 +500,8 @@ static pano_status solver_run(Solver<T>* S, int max_iterations, int every, const
         PANO_HIP(hipMemcpyAsync(&c->host_state[0], S->st, sizeof(SolverState), hipMemcpyDeviceToHost, c->stream));
         PANO_HIP(hipStreamSynchronize(c->stream));
         c->timer.solve = -1;
-        c->cl_solves += 1;
+        c->cl.ended(c->host_state[0].stalled != 0);
         if (!c->host_state[0].stalled) return PANO_OK;
-        c->cl_abandoned += 1;
         PANO_CHECK(start());
     }
     return solver_loop<T>(S, max_iterations, every, key, epi);
@@ -924,8 +923,8 @@ pano_status pano_precond_conjugate_gradient(pano_ctx ctx, const pano_grid* g, co
 pano_status pano_cg_cluster_counts(pano_ctx ctx, int64_t* solves, int64_t* abandoned) {
     Ctx* c = ctx_of(ctx);
     if (!c) return fail(PANO_ERR_INVALID, "ctx is null");
-    if (solves) *solves = c->cl_solves;
-    if (abandoned) *abandoned = c->cl_abandoned;
+    if (solves) *solves = c->cl.solves;
+    if (abandoned) *abandoned = c->cl.abandoned;
     return PANO_OK;
 }
 

@@ -412,6 +412,35 @@ static void abandoned(const char* what, const Dims& D, int chunk, int iterations
     g_late = Late();
 }
 
+// Solves of a context whose loops are all given up, then end again.
+static void use() {
+    ClusterUse u;
+    std::string seen;
+    for (int k = 0; k < 40; ++k) {
+        const bool t = u.take();
+        seen += t ? 'x' : '.';
+        if (t) u.ended(true);
+    }
+    int longest = 0, run = 0;
+    for (int k = 0; k < 10000; ++k) {
+        const bool t = u.take();
+        run = t ? 0 : run + 1;
+        longest = run > longest ? run : longest;
+        if (t) u.ended(true);
+    }
+    while (!u.take()) {
+    }
+    u.ended(false);
+    bool back = u.take();
+    u.ended(true);  // the first one again: no solve is left out
+    back = back && u.take();
+    ++runs;
+    if (seen != "xx.x...x.......x...............x........" || longest != 1023 || !back) {
+        ++fails;
+        printf("FAIL the solves that stay with the launches: %s, %d at most, back %d\n", seen.c_str(), longest, back);
+    }
+}
+
 int main() {
     cpu_set_t one;  // one thread runs at a time
     CPU_ZERO(&one);
@@ -422,6 +451,7 @@ int main() {
     orders<double>("3D Jacobi", Dims{17, 16, 17, 32}, 64, true, 4, 4);
     orders<double>("2D identity", Dims{1, 130, 64, 2}, 64, false, 3, 3);
     orders<float>("2D identity", Dims{1, 256, 64, 0}, 64, false, 2, 1);
+    use();
     abandoned<float>("few workgroups, long rows", Dims{1, 3, 300, 0}, 64, 3, 100);
     printf("%d orders, %d failures\n", runs, fails);
     return fails != 0;

@@ -68,6 +68,29 @@ def test_gpu_cluster_given_up_and_too_large(ctx, monkeypatch):
     monkeypatch.setenv("PANO_CG_CLUSTER", "0")
     assert np.array_equal(x1, cg(g))
     monkeypatch.delenv("PANO_CG_CLUSTER")
+    # once in a row: the next solve is one kernel again; it ends
+    x2, n = run(ctx, g, lambda: cg(g))
+    assert n == (1, 0) and np.array_equal(x2, x0)
     for dims in ((8, 2049), (1025, 1024)):  # a row too wide, too many cells
         big = grid(dims, (0,) * 6, "f4")
         assert run(ctx, big, lambda: cg(big, 3))[1] == (0, 0)
+
+
+def test_gpu_cluster_stays_with_the_launches(monkeypatch):
+    """Given up twice in a row, the next solve takes the launches, after three
+    times the next three; a context of its own, as its state lasts."""
+    own = pa.Context(0)
+    g = pa.Grid2d((257, 256), "f4", ctx=own)
+    seen = []
+    monkeypatch.setenv("PANO_CG_CLUSTER", "1")
+    for k in range(9):
+        x, n = run(own, g, lambda: cg(g, 20))
+        seen.append(n)
+        if k == 7:
+            monkeypatch.delenv("PANO_CG_CLUSTER")
+    up, no, ok = (1, 1), (0, 0), (1, 0)
+    assert seen == [up, up, no, up, no, no, no, up, no]  # the eighth: four in a row
+    for _ in range(6):
+        assert run(own, g, lambda: cg(g, 20))[1] == no
+    assert run(own, g, lambda: cg(g, 20))[1] == ok  # back to one kernel
+    assert run(own, g, lambda: cg(g, 20))[1] == ok
