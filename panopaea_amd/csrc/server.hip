@@ -10,20 +10,16 @@
 // over every admitted request. The launches of each phase go through
 // BatchCore, so a request's arithmetic and reduction order are those of the
 // request alone.
-#include <sys/mman.h>
-
 #include <algorithm>
 #include <chrono>
-#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <map>
 #include <memory>
-#include <system_error>
-#include <thread>
 #include <unordered_map>
 
 #include "batch.hpp"
+#include "host_pool.hpp"
 
 namespace pano {
 
@@ -71,90 +67,6 @@ public:
 private:
     std::map<int64_t, int64_t> free_;
     int64_t used_ = 0;
-};
-
-// memcpy of large host ranges by a few threads. One thread copies into memory
-// it touches for the first time at 10 to 14 GB/s (page faults), four at three
-// times that. Threads that cannot be started leave their part to the caller.
-constexpr size_t kParCopyMin = size_t(4) << 20;
-static void par_copy(char* dst, const char* src, size_t n) {
-    constexpr int N = 4;
-    if (n < kParCopyMin) {
-        memcpy(dst, src, n);
-        return;
-    }
-    const size_t part = ((n / N + 4095) / 4096) * 4096;
-    std::thread th[N - 1];
-    for (int i = 1; i < N; ++i) {
-        const size_t a = std::min(n, i * part), b = i == N - 1 ? n : std::min(n, (i + 1) * part);
-        try {
-            th[i - 1] = std::thread([=] { memcpy(dst + a, src + a, b - a); });
-        } catch (const std::system_error&) {
-            memcpy(dst + a, src + a, b - a);
-        }
-    }
-    memcpy(dst, src, std::min(n, part));
-    for (std::thread& t : th)
-        if (t.joinable()) t.join();
-}
-
-// Host blocks for the velocities of queued requests. A block that a request
-// gives back is kept for the next one, up to kKeep bytes: a new allocation of
-// this size is page faults on its first write (the copy at submit took 190 ms
-// for 0.9 GB into new vectors). Blocks are huge-page advised.
-class HostPool {
-public:
-    ~HostPool() {
-        for (auto& b : free_) ::free(b.second);
-    }
-    // a block of at least n bytes (nullptr: no memory); *cap its size
-    void* take(size_t n, size_t* cap) {
-        auto it = free_.lower_bound(n);
-        if (it != free_.end() && it->first <= 2 * n + kAlign) {
-            void* p = it->second;
-            *cap = it->first;
-            kept_ -= it->first;
-            free_.erase(it);
-            return p;
-        }
-        *cap = (n + kAlign - 1) / kAlign * kAlign;
-        void* p = nullptr;
-        if (posix_memalign(&p, kAlign, *cap) != 0) return nullptr;
-        (void)madvise(p, *cap, MADV_HUGEPAGE);
-        return p;
-    }
-    void give(void* p, size_t cap) {
-        if (kept_ + cap > kKeep) {
-            ::free(p);
-            return;
-        }
-        kept_ += cap;
-        free_.emplace(cap, p);
-    }
-
-private:
-    static constexpr size_t kAlign = size_t(2) << 20, kKeep = size_t(1) << 30;
-    std::multimap<size_t, void*> free_;
-    size_t kept_ = 0;
-};
-
-// A block of the pool, given back when it goes.
-struct HostBlock {
-    HostPool* pool = nullptr;
-    void* p = nullptr;
-    size_t cap = 0;
-    HostBlock() = default;
-    HostBlock(HostPool* pl, size_t n) : pool(pl) { p = pl->take(n, &cap); }
-    HostBlock(HostBlock&& o) noexcept : pool(o.pool), p(o.p), cap(o.cap) { o.p = nullptr; }
-    HostBlock& operator=(HostBlock&& o) noexcept {
-        std::swap(pool, o.pool);
-        std::swap(p, o.p);
-        std::swap(cap, o.cap);
-        return *this;
-    }
-    ~HostBlock() {
-        if (p) pool->give(p, cap);
-    }
 };
 
 struct Request {
