@@ -8,7 +8,6 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
-#include <system_error>
 #include <thread>
 
 namespace pano {
@@ -29,7 +28,7 @@ inline void par_copy(char* dst, const char* src, size_t n) {
         const size_t a = std::min(n, i * part), b = i == N - 1 ? n : std::min(n, (i + 1) * part);
         try {
             th[i - 1] = std::thread([=] { memcpy(dst + a, src + a, b - a); });
-        } catch (const std::system_error&) {
+        } catch (...) {  // no thread, or no memory for one
             memcpy(dst + a, src + a, b - a);
         }
     }
@@ -71,8 +70,13 @@ public:
             ::free(p);
             return;
         }
+        try {
+            free_.emplace(cap, p);
+        } catch (...) {  // no memory to remember it by (destructors call this)
+            ::free(p);
+            return;
+        }
         kept_ += cap;
-        free_.emplace(cap, p);
     }
 
 private:

@@ -243,8 +243,9 @@ static pano_status admit_at(Server* S, Request* r, int64_t off, std::vector<Requ
     PANO_CHECK(stage_upload(S, S->core_all.cfgs + r->slot, &cf, sizeof(SolveCfg)));
     float* u = reinterpret_cast<float*>(S->arena + r->g.o_u[0]);
     if (r->faces.p) {
+        S->uploading.emplace_back();  // room for the block before a copy reads it
         PANO_HIP(hipMemcpyAsync(u, r->faces.p, r->g.faces * sizeof(float), hipMemcpyHostToDevice, c->stream));
-        S->uploading.push_back(std::move(r->faces));
+        S->uploading.back() = std::move(r->faces);
     } else {
         double* dtab = reinterpret_cast<double*>(S->arena + r->tab_off);
         PANO_CHECK(stage_upload(S, dtab, r->gen_tab.data(), r->gen_tab.size() * sizeof(double)));

@@ -1,11 +1,24 @@
 // The server's host blocks (host_pool.hpp): what a request of a size holds,
 // what it is given back, and how much the pool keeps.
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
+#include <new>
 #include <vector>
 
 #include "host_pool.hpp"
 using namespace pano;
+
+// operator new fails while g_fail_from counts down to 0 and after
+static std::atomic<int> g_fail_from{1 << 30};
+void* operator new(size_t n) {
+    if (g_fail_from.fetch_sub(1) <= 0) throw std::bad_alloc();
+    void* p = malloc(n ? n : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 static int fails = 0;
 #define CHECK(cond, ...)                 \
@@ -70,6 +83,26 @@ int main() {
         for (size_t i = 0; i < n; ++i) a[i] = (unsigned char)(i * 131 + (i >> 9));
         par_copy((char*)b.data(), (const char*)a.data(), n);
         CHECK(memcmp(a.data(), b.data(), n) == 0 && b[n] == 7, "copy of %zu bytes", n);
+    }
+    // no host memory for a thread's start: the copy is whole all the same
+    for (int k = 0; k < 3; ++k) {
+        const size_t n = kParCopyMin + 777;
+        std::vector<char> a(n, 3), b(n, 0);
+        g_fail_from = k;
+        par_copy(b.data(), a.data(), n);
+        g_fail_from = 1 << 30;
+        CHECK(a == b, "copy with %d allocations left", k);
+    }
+    // none for the pool's own record: the block is freed, not kept
+    {
+        HostPool P;
+        {
+            HostBlock b(&P, 5000);
+            g_fail_from = 0;
+        }
+        g_fail_from = 1 << 30;
+        HostBlock c(&P, 5000);
+        CHECK(c.p != nullptr, "no block");
     }
     printf("%d failures\n", fails);
     return fails != 0;
