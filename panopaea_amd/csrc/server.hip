@@ -19,6 +19,7 @@
 #include <unordered_map>
 
 #include "batch.hpp"
+#include "fetch_stage.hpp"
 #include "host_pool.hpp"
 
 namespace pano {
@@ -92,8 +93,7 @@ struct Server {
     RangeAlloc alloc;
     HostPool pool;                      // outlives the requests below
     std::vector<HostBlock> uploading;   // blocks whose upload the stream may still read
-    char* fetch_stage = nullptr;        // pinned, two halves of kFetchChunk bytes
-    hipEvent_t fetch_ev[2] = {nullptr, nullptr};
+    FetchStage fetch;
     BatchCore core_all, core_new, core_done;
     SolverState* hstates = nullptr;  // pinned
     std::vector<SolveCfg> hcfg;
@@ -150,19 +150,11 @@ __global__ __launch_bounds__(256) void k_rb_to_nat(Dims D, Grid3 G, float* dst, 
 
 // Device range to (pageable) host memory. Large ranges go through two pinned
 // halves: the next chunk's copy runs while a few threads move the last one to
-// its place (a plain copy into new memory: 10 GB/s).
-constexpr size_t kFetchChunk = size_t(8) << 20;
+// its place (a plain copy into new memory, also taken where there are no such
+// halves: 10 GB/s).
 static pano_status fetch_range(Server* S, char* dst, const char* src, size_t n) {
     hipStream_t st = S->c->stream;
-    if (n >= kParCopyMin && !S->fetch_stage) {
-        if (hipHostMalloc((void**)&S->fetch_stage, 2 * kFetchChunk) != hipSuccess) {
-            (void)hipGetLastError();
-            S->fetch_stage = nullptr;
-            return fail(PANO_ERR_OOM, "pinned staging of %zu bytes", 2 * kFetchChunk);
-        }
-        for (hipEvent_t& e : S->fetch_ev) PANO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
-    if (n < kParCopyMin) {
+    if (n < kParCopyMin || !S->fetch.make()) {
         PANO_HIP(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
         PANO_HIP(hipStreamSynchronize(st));
         return PANO_OK;
@@ -170,16 +162,16 @@ static pano_status fetch_range(Server* S, char* dst, const char* src, size_t n) 
     const size_t chunks = (n + kFetchChunk - 1) / kFetchChunk;
     auto size_of = [&](size_t k) { return std::min(kFetchChunk, n - k * kFetchChunk); };
     auto enqueue = [&](size_t k) -> pano_status {
-        PANO_HIP(hipMemcpyAsync(S->fetch_stage + (k & 1) * kFetchChunk, src + k * kFetchChunk, size_of(k),
+        PANO_HIP(hipMemcpyAsync(S->fetch.p + (k & 1) * kFetchChunk, src + k * kFetchChunk, size_of(k),
                                 hipMemcpyDeviceToHost, st));
-        PANO_HIP(hipEventRecord(S->fetch_ev[k & 1], st));
+        PANO_HIP(hipEventRecord(S->fetch.ev[k & 1], st));
         return PANO_OK;
     };
     PANO_CHECK(enqueue(0));
     for (size_t k = 0; k < chunks; ++k) {
         if (k + 1 < chunks) PANO_CHECK(enqueue(k + 1));
-        PANO_HIP(hipEventSynchronize(S->fetch_ev[k & 1]));
-        par_copy(dst + k * kFetchChunk, S->fetch_stage + (k & 1) * kFetchChunk, size_of(k));
+        PANO_HIP(hipEventSynchronize(S->fetch.ev[k & 1]));
+        par_copy(dst + k * kFetchChunk, S->fetch.p + (k & 1) * kFetchChunk, size_of(k));
     }
     return PANO_OK;
 }
@@ -413,9 +405,6 @@ pano_status pano_server_destroy(pano_server h) {
     if (S->arena) (void)hipFree(S->arena);
     if (S->hstates) (void)hipHostFree(S->hstates);
     if (S->stage) (void)hipHostFree(S->stage);
-    if (S->fetch_stage) (void)hipHostFree(S->fetch_stage);
-    for (hipEvent_t e : S->fetch_ev)
-        if (e) (void)hipEventDestroy(e);
     delete h;
     return PANO_OK;
 }
