@@ -25,9 +25,10 @@ struct SolveCfg {
 
 // Reduces the FP64 partials part0[0..np) (+ part1[0..np) when part1 is not
 // null) in a fixed order and applies `op` to the solver state. Run by one
-// one-dimensional workgroup of NT threads (all of them), 256 up to kFinSmall partials:
-// a few thousand partials are one round of loads for 256 threads, whose four
-// waves are started and combined faster than sixteen. The state is read once, at the
+// one-dimensional workgroup of NT threads (all of them): 256 for a few thousand
+// partials (kFinSmall for one grid; a batch's limit is its own), which are one or
+// a few rounds of loads for four waves that are started and combined faster than
+// sixteen; 1024 past that. The state is read once, at the
 // start, and the done test comes at the end, after the reduction (the
 // partials' loads no longer wait for it): a finished solve (done) changes
 // nothing; its partials are read and left unused.
