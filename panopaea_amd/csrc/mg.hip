@@ -428,7 +428,9 @@ static pano_status eig1d(int n, int lo, int hi, std::vector<double>& V, std::vec
     return PANO_OK;
 }
 
-// Device copy of the eigenbasis of one axis, cached per (n, lo, hi).
+// Device copy of the eigenbasis of one axis, cached per (n, lo, hi): V, followed
+// by its transpose (basis_t), which the matrix products read row by row where V
+// would be read column by column.
 pano_status axis_basis(Ctx* c, int n, int lo, int hi, double** V, double** lam) {
     char key[64];
     snprintf(key, sizeof(key), "eig:%d:%d:%d", n, lo, hi);
@@ -437,17 +439,24 @@ pano_status axis_basis(Ctx* c, int n, int lo, int hi, double** V, double** lam) 
         std::vector<double> hv, hl;
         PANO_CHECK(eig1d(n, lo, hi, hv, hl));
         void* p = nullptr;
-        size_t bytes = ((size_t)n * n + n) * sizeof(double);
+        const size_t nn = (size_t)n * n;
+        std::vector<double> all(2 * nn + n);  // V, its transpose, the eigenvalues
+        for (int j = 0; j < n; ++j)
+            for (int k = 0; k < n; ++k) {
+                all[(size_t)j * n + k] = hv[(size_t)j * n + k];
+                all[nn + (size_t)k * n + j] = hv[(size_t)j * n + k];
+            }
+        std::copy(hl.begin(), hl.end(), all.begin() + 2 * nn);
+        const size_t bytes = all.size() * sizeof(double);
         if (hipMalloc(&p, bytes) != hipSuccess) {
             (void)hipGetLastError();
             return fail(PANO_ERR_OOM, "eigenbasis allocation failed");
         }
-        PANO_HIP(hipMemcpy(p, hv.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice));
-        PANO_HIP(hipMemcpy((double*)p + (size_t)n * n, hl.data(), n * sizeof(double), hipMemcpyHostToDevice));
+        PANO_HIP(hipMemcpy(p, all.data(), bytes, hipMemcpyHostToDevice));
         it = c->consts.emplace(key, p).first;
     }
     *V = (double*)it->second;
-    *lam = (double*)it->second + (size_t)n * n;
+    *lam = (double*)it->second + 2 * (size_t)n * n;
     return PANO_OK;
 }
 
@@ -618,16 +627,23 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_zcol(int nx, int ny, int nz
 //  inverse: plane K, 16 rows j: y for them (every column), then x.
 // 64^3 53 + 28 + 49 us with a sum per thread, 7 + 7 + 9 now; 32^3 6.4 + 5.8 +
 // 5.4, now 4.6 + 4.6 + 4.8 (launch and two rounds of loads).
-constexpr int kFdm3Threads = 256;
+// An axis past 64 cells has 16 waves per workgroup instead of four, a tile each;
+// and where that leaves few workgroups their long products are split, or one
+// workgroup's CU reads the whole basis: y forward below 64 workgroups, z up to
+// 128. Two-level V-cycles, us, with a sum per thread / four waves / now: coarsest
+// level 256 x 8 x 8 (z, y, x) 75 / 91 / 55, 8 x 256 x 8 69 / 81 / 58, 7 x 4 x 248
+// 56 / 59 / 53, 256 x 32 x 32 263 / 135 / 93, 128^3 2147 / 380 / 339. (256 x 48 x
+// 48, 144 workgroups in z: 157 not split, 154 split, f64 215 and 221.)
+__device__ __forceinline__ const double* basis_t(const double* V, int n) { return V + (size_t)n * n; }
 constexpr int kFdm3P = 17;  // row length in LDS of a block of 16 columns
 inline size_t fdm3_lds_cols(int n) { return (size_t)((n + 15) / 16 * 16) * kFdm3P * sizeof(double); }
 __host__ __device__ inline int fdm3_row(int nx) { return (nx + 15) / 16 * 16 + 2; }
 
-// forward x then y of plane K, columns [i0, i0 + 16): in -> out (double)
-template <typename Tin>
-__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_fwd(int nx, int ny, const Tin* in, double* out,
-                                                           const double* Vx, const double* Vy,
-                                                           const SolverState* st) {
+// forward x then y of plane K, columns [i0, i0 + 16): in -> out (double); the
+// rows of y, with the whole x product before them, may be split over gridDim.y
+template <typename Tin, int NT>
+__global__ __launch_bounds__(NT) void k_fdm3_fwd(int nx, int ny, const Tin* in, double* out, const double* Vx,
+                                                 const double* Vy, const SolverState* st) {
     if (st->done) return;
     extern __shared__ double fdm_lds[];
     const int gx = (nx + 15) >> 4, K = blockIdx.x / gx, i0 = (blockIdx.x - K * gx) * 16;
@@ -635,7 +651,7 @@ __global__ __launch_bounds__(kFdm3Threads) void k_fdm3_fwd(int nx, int ny, const
     const int ic = imin(i0 + r, nx - 1);
     const Tin* src = in + (int64_t)K * nx * ny;
     double* dst = out + (int64_t)K * nx * ny;
-    for (int jt = w; jt < gy; jt += kFdm3Threads / 64) {
+    for (int jt = w; jt < gy; jt += NT / 64) {
         const int jc = imin(jt * 16 + r, ny - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
         mfma_tile<8>(0, nx, [&](int q) { return (double)src[jc * nx + q]; }, [&](int q) { return Vx[q * nx + ic]; },
@@ -644,7 +660,8 @@ __global__ __launch_bounds__(kFdm3Threads) void k_fdm3_fwd(int nx, int ny, const
         for (int v = 0; v < 4; ++v) fdm_lds[(jt * 16 + 4 * v + h) * kFdm3P + r] = acc[v];
     }
     __syncthreads();
-    for (int jt = w; jt < gy; jt += kFdm3Threads / 64) {
+    const int jn = (gy + gridDim.y - 1) / gridDim.y, j0 = blockIdx.y * jn, j1 = imin(j0 + jn, gy);
+    for (int jt = j0 + w; jt < j1; jt += NT / 64) {
         const int jc = imin(jt * 16 + r, ny - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
         mfma_tile<8>(0, ny, [&](int q) { return Vy[q * ny + jc]; }, [&](int q) { return fdm_lds[q * kFdm3P + r]; },
@@ -659,15 +676,17 @@ __global__ __launch_bounds__(kFdm3Threads) void k_fdm3_fwd(int nx, int ny, const
 
 // cells [e0, e0 + 16) of every plane: z forward, divide by s*(lx+ly+lz) (0 on
 // the null space), z inverse, in place on data (double)
-__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_z(int nx, int ny, int nz, double* data, const double* Vz,
-                                                         const double* lx, const double* ly, const double* lz,
-                                                         double s, double eps, const SolverState* st) {
+template <int NT>
+__global__ __launch_bounds__(NT) void k_fdm3_z(int nx, int ny, int nz, double* data, const double* Vz,
+                                               const double* lx, const double* ly, const double* lz, double s,
+                                               double eps, const SolverState* st) {
     if (st->done) return;
     extern __shared__ double fdm_lds[];
     const int P = nx * ny, lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4;
     const int e = blockIdx.x * 16 + r, ec = imin(e, P - 1), gz = (nz + 15) >> 4;
     const double lxy = lx[ec % nx] + ly[ec / nx];
-    for (int kt = w; kt < gz; kt += kFdm3Threads / 64) {
+    const double* Wz = basis_t(Vz, nz);
+    for (int kt = w; kt < gz; kt += NT / 64) {
         const int kc = imin(kt * 16 + r, nz - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
         mfma_tile<8>(0, nz, [&](int q) { return Vz[q * nz + kc]; }, [&](int q) { return data[(int64_t)q * P + ec]; },
@@ -680,10 +699,10 @@ __global__ __launch_bounds__(kFdm3Threads) void k_fdm3_z(int nx, int ny, int nz,
         }
     }
     __syncthreads();
-    for (int kt = w; kt < gz; kt += kFdm3Threads / 64) {
+    for (int kt = w; kt < gz; kt += NT / 64) {
         const int kc = imin(kt * 16 + r, nz - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
-        mfma_tile<8>(0, nz, [&](int q) { return Vz[kc * nz + q]; }, [&](int q) { return fdm_lds[q * kFdm3P + r]; },
+        mfma_tile<8>(0, nz, [&](int q) { return Wz[q * nz + kc]; }, [&](int q) { return fdm_lds[q * kFdm3P + r]; },
                      acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -693,30 +712,58 @@ __global__ __launch_bounds__(kFdm3Threads) void k_fdm3_z(int nx, int ny, int nz,
     }
 }
 
-// inverse y then x of plane K, rows [j0, j0 + 16): in (double) -> out
-template <typename Tout>
-__global__ __launch_bounds__(kFdm3Threads) void k_fdm3_inv(int nx, int ny, const double* in, Tout* out,
-                                                           const double* Vx, const double* Vy,
-                                                           const SolverState* st) {
+// The z pass as two launches (INV: the inverse), 64 planes of 16 cells per
+// workgroup: for long columns of few cells, which would leave both products of
+// a column, and all of the basis, to one CU.
+template <bool INV>
+__global__ __launch_bounds__(256) void k_fdm3_z_part(int nx, int ny, int nz, const double* in, double* out,
+                                                     const double* Vz, const double* lx, const double* ly,
+                                                     const double* lz, double s, double eps, const SolverState* st) {
+    if (st->done) return;
+    const int P = nx * ny, lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4;
+    const int e = blockIdx.x * 16 + r, ec = imin(e, P - 1), k0 = blockIdx.y * 64 + 16 * w;
+    if (k0 >= nz) return;
+    const int kc = imin(k0 + r, nz - 1);
+    const double* W = INV ? basis_t(Vz, nz) : Vz;
+    const double lxy = lx[ec % nx] + ly[ec / nx];
+    mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
+    mfma_tile<8>(0, nz, [&](int q) { return W[q * nz + kc]; }, [&](int q) { return in[(int64_t)q * P + ec]; }, acc);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const int k = k0 + 4 * v + h;
+        const double lam = lxy + lz[imin(k, nz - 1)];
+        if (k < nz && e < P) out[(int64_t)k * P + e] = INV ? acc[v] : lam > eps ? acc[v] / (s * lam) : 0.0;
+    }
+}
+
+// inverse y then x of plane K, rows [j0, j0 + 16): in (double) -> out. One tile
+// of columns is one wave's chain of loads in y: twice as many in flight then.
+template <typename Tout, int NT>
+__global__ __launch_bounds__(NT) void k_fdm3_inv(int nx, int ny, const double* in, Tout* out, const double* Vx,
+                                                 const double* Vy, const SolverState* st) {
     if (st->done) return;
     extern __shared__ double fdm_lds[];
     const int gy = (ny + 15) >> 4, K = blockIdx.x / gy, j0 = (blockIdx.x - K * gy) * 16, R = fdm3_row(nx);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = lane & 15, h = lane >> 4, gx = (nx + 15) >> 4;
     const int jc = imin(j0 + r, ny - 1);
+    const double *Wx = basis_t(Vx, nx), *Wy = basis_t(Vy, ny);
     const double* src = in + (int64_t)K * nx * ny;
     Tout* dst = out + (int64_t)K * nx * ny;
-    for (int it = w; it < gx; it += kFdm3Threads / 64) {
+    for (int it = w; it < gx; it += NT / 64) {
         const int ic = imin(it * 16 + r, nx - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
-        mfma_tile<8>(0, ny, [&](int q) { return Vy[jc * ny + q]; }, [&](int q) { return src[q * nx + ic]; }, acc);
+        auto fa = [&](int q) { return Wy[q * ny + jc]; };
+        auto fb = [&](int q) { return src[q * nx + ic]; };
+        if (gx == 1 && ny > 64) mfma_tile<16>(0, ny, fa, fb, acc);
+        else mfma_tile<8>(0, ny, fa, fb, acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) fdm_lds[(4 * v + h) * R + it * 16 + r] = acc[v];
     }
     __syncthreads();
-    for (int it = w; it < gx; it += kFdm3Threads / 64) {
+    for (int it = w; it < gx; it += NT / 64) {
         const int ic = imin(it * 16 + r, nx - 1);
         mfma_d4 acc = {0.0, 0.0, 0.0, 0.0};
-        mfma_tile<8>(0, nx, [&](int q) { return fdm_lds[r * R + q]; }, [&](int q) { return Vx[ic * nx + q]; }, acc);
+        mfma_tile<8>(0, nx, [&](int q) { return fdm_lds[r * R + q]; }, [&](int q) { return Wx[q * nx + ic]; }, acc);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int j = j0 + 4 * v + h, i = it * 16 + r;
@@ -856,13 +903,37 @@ static pano_status coarse_solve(Ctx* c, MG<T>* m, T* z, const T* r, const Solver
             PANO_HIP(hipGetLastError());
             return PANO_OK;
         }
+        const std::integral_constant<int, 256> nt4{};    // four waves: one tile each up to 64 cells per axis
+        const std::integral_constant<int, 1024> nt16{};  // 16 for longer axes
         const unsigned gx = (unsigned)((nx + 15) / 16), gy = (unsigned)((ny + 15) / 16);
-        hipLaunchKernelGGL((k_fdm3_fwd<T>), dim3(nz * gx), dim3(kFdm3Threads), fdm3_lds_cols(ny), S, nx, ny, r, t0, Vx,
-                           Vy, st);
-        hipLaunchKernelGGL(k_fdm3_z, dim3((nx * ny + 15) / 16), dim3(kFdm3Threads), fdm3_lds_cols(nz), S, nx, ny, nz,
-                           t0, Vz, lx, ly, lz, s, eps, st);
-        hipLaunchKernelGGL((k_fdm3_inv<T>), dim3(nz * gy), dim3(kFdm3Threads),
-                           (size_t)16 * fdm3_row(nx) * sizeof(double), S, nx, ny, (const double*)t0, z, Vx, Vy, st);
+        const unsigned gz = (unsigned)((nz + 15) / 16), P16 = (unsigned)((nx * ny + 15) / 16);
+        auto fwd = [&](auto nt, unsigned split) {
+            hipLaunchKernelGGL((k_fdm3_fwd<T, nt.value>), dim3(nz * gx, split), dim3(nt.value), fdm3_lds_cols(ny), S, nx,
+                               ny, r, t0, Vx, Vy, st);
+        };
+        auto zz = [&](auto nt) {
+            hipLaunchKernelGGL(k_fdm3_z<nt.value>, dim3(P16), dim3(nt.value), fdm3_lds_cols(nz), S, nx, ny, nz, t0, Vz,
+                               lx, ly, lz, s, eps, st);
+        };
+        auto inv = [&](auto nt) {
+            hipLaunchKernelGGL((k_fdm3_inv<T, nt.value>), dim3(nz * gy), dim3(nt.value),
+                               (size_t)16 * fdm3_row(nx) * sizeof(double), S, nx, ny, (const double*)t0, z, Vx, Vy, st);
+        };
+        if (gy <= 4) fwd(nt4, 1);
+        else fwd(nt16, nz * gx < 64 ? (gy + 3) / 4 : 1);
+        if (gz <= 4) {
+            zz(nt4);
+        } else if (P16 > 128) {
+            zz(nt16);
+        } else {
+            const dim3 zg(P16, (gz + 3) / 4);
+            hipLaunchKernelGGL(k_fdm3_z_part<false>, zg, dim3(256), 0, S, nx, ny, nz, (const double*)t0, t1, Vz, lx, ly,
+                               lz, s, eps, st);
+            hipLaunchKernelGGL(k_fdm3_z_part<true>, zg, dim3(256), 0, S, nx, ny, nz, (const double*)t1, t0, Vz, lx, ly,
+                               lz, s, eps, st);
+        }
+        if (gx <= 4) inv(nt4);
+        else inv(nt16);
         PANO_HIP(hipGetLastError());
         return PANO_OK;
     }
