@@ -47,16 +47,19 @@ struct AdvShape {
 };
 
 // Workgroup chunks: tiles of TX x TY cells by chunks of zc planes, halved down
-// to 2 while the launch has fewer than `want` workgroups.
+// to 2 while the launch has fewer than `want` workgroups, and (single) to one
+// plane below 5/8 of that.
 struct AdvGrid {
     int gx, gy, zc, nch, nb;
 };
 template <int TX, int TY>
-inline AdvGrid adv_grid(const Dims& D, int zc, int want = 0) {
+inline AdvGrid adv_grid(const Dims& D, int zc, int want = 0, bool single = false) {
     AdvGrid g;
     g.gx = (D.w + TX - 1) / TX;
     g.gy = (D.h + TY - 1) / TY;
-    while (zc > 2 && (int64_t)g.gx * g.gy * ((D.d + zc - 1) / zc) < want) zc /= 2;
+    const auto nb = [&] { return (int64_t)g.gx * g.gy * ((D.d + zc - 1) / zc); };
+    while (zc > 2 && nb() < want) zc /= 2;
+    if (single && zc == 2 && nb() < want * 5 / 8) zc = 1;
     g.zc = zc < D.d ? zc : D.d;
     g.nch = (D.d + g.zc - 1) / g.zc;
     g.nb = g.gx * g.gy * g.nch;

@@ -265,13 +265,20 @@ bool advect_fused_on(const Dims& D) {
 // against 233 as 64 x 8: less halo), or of 64 x 8 where those cover the plane
 // with fewer cells outside it (40 x 40 planes: 12.5 us against 16.3). Chunks of
 // 16 planes, shorter while there are fewer than 512 workgroups (64^3 step: 61 us
-// with 32 workgroups, 14 with 256).
+// with 32 workgroups, 14 with 256); for the faces alone, with fewer than 320 of
+// two planes each, the chain of a workgroup is what counts and a single plane is
+// shorter (with the density 64^3 steps took 648 us so, 644 with two planes). Faces,
+// us a call with two planes / one, displacements of up to 1 and 3 cells; three
+// launches per component took 9.3 at 30^3, 13.3 and 14.3 at 136 x 57 x 20:
+//   30^3 (60 workgroups of two planes) 9.5 / 6.4 and 10.4 / 6.8;
+//   136 x 57 x 20 (272) 11.9 / 11.5 and 14.5 / 12.1;
+//   60 x 99 x 53 (378) 12.3 / 13.9 and 16.3 / 16.6.
 template <bool DENS>
 static void launch_fused(Ctx* c, const char* name, double bytes, const Dims& D, float* rho_out, const float* rho_in,
                          float* vel_out, const float* vel_in, double dt, double buoy_c, const double* src_sphere) {
     auto go = [&](auto tx, auto ty) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value;
-        const AdvGrid g = adv_grid<TX, TY>(D, 16, 512);
+        const AdvGrid g = adv_grid<TX, TY>(D, 16, 512, !DENS);
         klaunch(c, name, bytes, k_advect_fused<TX, TY, DENS>, dim3(g.nb), dim3(TX * TY), D, g, split_faces(D, vel_in),
                 rho_in, split_faces(D, vel_out), rho_out, make_sphere(src_sphere), (float)dt, (float)buoy_c);
     };
