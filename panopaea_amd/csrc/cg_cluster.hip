@@ -282,12 +282,6 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
         if (!got || !kept) flag = 0;
         __syncthreads();
         if (!flag) break;
-        // only now have the waves together seen every p.q: a wave has seen its own slots'
-        if (t < kClCopies) {
-            st_agent(&S[t].pq[(k + 3) & 3][g], kClEmpty);
-            st_agent(&S[t].zr[k2 ^ 1][g], kClEmpty);
-            st_agent(&S[t].mx[k2 ^ 1][g], kClEmpty);
-        }
         pq = waves_all<ClSum, NW>(red[1][0]);
         alpha = sigma / pq;
         if (!(alpha == alpha) || fabs(alpha) > 1.7e308) {
@@ -323,6 +317,12 @@ __global__ __launch_bounds__(NT) void k_cg_cluster(Dims D, int n, int chunk, T* 
         if (t < kClCopies) {
             st_agent(&S[t].zr[k2][g], cl_bits(waves_all<ClSum, NW>(red[0][0])));
             st_agent(&S[t].mx[k2][g], cl_bits(waves_all<ClMax, NW>(red[0][1])));
+            // behind the barrier of the p.q exchange, at which the waves together had
+            // seen every p.q (a wave has seen its own slots' only), and behind the
+            // values that others wait for
+            st_agent(&S[t].pq[(k + 3) & 3][g], kClEmpty);
+            st_agent(&S[t].zr[k2 ^ 1][g], kClEmpty);
+            st_agent(&S[t].mx[k2 ^ 1][g], kClEmpty);
         }
         got = cl_poll<2>(S[mr].zr[k2], S[mr].mx[k2], &S->stop, P, spin, v);
         s = wave_all<ClSum>(v[0]);
