@@ -74,8 +74,14 @@ pano_status pano_fill_zero(pano_ctx ctx, void* dst, size_t bytes); /* fill kerne
  * context's stream until pano_timer_stop, which returns the summed duration,
  * the launch count (launches the solver's converged flag made no-ops are
  * excluded) and the kernel's algorithmic bytes per launch. Names:
- * "smooth_l0", "apply_dot", "update", "residual_l0", "restrict_l0",
- * "prolong_l0", "advect_mac", "advect", "project", "neg_div". */
+ * "apply_dot", "update", "search", "dot", "advect" and "advect_fused" (3D f32
+ * steps), "advect_mac" (3D f32, a velocity by itself); of multigrid's level 0,
+ * by the form its size and type take: "smooth_l0", "smooth_first_l0",
+ * "red_init_l0", "residual_l0", "restrict_l0", "prolong_l0" (separate passes),
+ * "smooth_pre_l0", "smooth_post_l0", "resrestrict_l0" (one-pass levels),
+ * "leg_down_l0", "leg_up_l0" (below 2^20 cells). A kernel that does not run has
+ * no launches. While a timer runs, small solves take their separate launches
+ * instead of one kernel (pano_cg_cluster_counts). */
 pano_status pano_timer_start(pano_ctx ctx, const char* kernel);
 pano_status pano_timer_stop(pano_ctx ctx, double* total_ms, int64_t* launches, double* bytes_per_launch);
 const char* pano_status_string(pano_status s);
@@ -176,7 +182,8 @@ pano_status pano_precond_conjugate_gradient(pano_ctx, const pano_grid*, const pa
 /* No reference counterpart. Identity and Jacobi solves (and steps) of small
  * grids run their CG loop as one kernel whose workgroups wait for each other;
  * where they do not all get to run (the device is shared), the kernel gives up
- * and the solve runs again as separate launches. Counts of this context: the
+ * and the solve runs again as separate launches, whose sums are added in another
+ * order. Counts of this context: the
  * solves begun that way and those of them given up (either pointer may be
  * null). After two in a row that were given up the next solve takes the
  * launches at once, after three the next three, and so on up to 1023, until one
